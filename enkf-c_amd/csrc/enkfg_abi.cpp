@@ -106,13 +106,16 @@ struct enkfg_ctx {
     std::vector<short> otype, ostatus;
     std::vector<float> olon, olat, oestd;
     bool obs_set = false;
-    DevBuf d_nodes, d_types, d_obsids, d_type, d_status, d_estd, d_sqrtrf, d_perm;
+    DevBuf d_nodes, d_noderow, d_types, d_obsids, d_type, d_status, d_estd, d_sqrtrf, d_perm, d_xyz, d_boxes;
     std::vector<TypeInfo> tinfo;
-    // Device rows of S, s and status are ordered by tree preorder (type by
-    // type), so the obs a node's range search returns -- a few subtrees --
-    // are a few runs of nearby rows; perm[row] is the observation index.
-    // kd nodes and the local lists hold rows; the API speaks obs indices.
+    // Device rows of S, s and status are ordered along a Morton curve (type by
+    // type), so the obs near a node are a few runs of nearby rows; perm[row]
+    // is the observation index.  The local lists hold rows; the API speaks
+    // obs indices.
     std::vector<int> perm;
+    size_t nsearch = 0;           // rows that are searched (the types' rows come first)
+    bool box_ok = false;          // finite coordinates only: the box search applies
+    bool trees_built = false;     // d_nodes, d_noderow hold the reference's trees
 
     // S and s
     DevBuf d_S, d_s, d_tmp, d_tmp2;
@@ -124,11 +127,10 @@ struct enkfg_ctx {
     int node_geo = 0;
     DevBuf d_qxyz, d_glob, d_vis, d_counts, d_offsets, d_scantmp, d_ids, d_lc;
     DevBuf d_raw, d_rawoff, d_rrow, d_rd2, d_srow, d_sd2;   // NLOBSMAX candidates
-    // one-walk localisation: chunk pool (capacity from the last two-walk
-    // localisation), list heads, pool counter and overflow flag
-    DevBuf d_heads, d_cids, d_clc, d_cnext, d_lflag;
-    long long pool_cap = 0;
+    DevBuf d_lflag;               // box search: an obs lies at exactly a radius
     bool lists_valid = false;
+    bool lists_ordered = false;   // the lists are in the reference's order
+    bool lists_vis = false;       // they were made with the visibility mask in d_vis
 
     // calc batching: nodes ordered by obs-count bucket (heaviest first), and
     // the autotuned Gram tile groups per [precision][bucket] (0 = not tuned)
@@ -195,6 +197,83 @@ int fail(enkfg_ctx* c, int code, const char* fmt, ...)
             return fail((c), (e_ == hipErrorOutOfMemory) ? ENKFG_ERR_NOMEM : ENKFG_ERR_HIP, "%s: %s (%s:%d)", \
                         #expr, hipGetErrorString(e_), __FILE__, __LINE__);                                 \
     } while (0)
+
+// 3D chord coordinates (geographic types) or (lon, lat, 0) of an observation
+void obs_coords(const enkfg_ctx* c, int i, bool geographic, double* out)
+{
+    if (geographic) {
+        ll2xyz((double)c->olon[i], (double)c->olat[i], out);
+    } else {
+        out[0] = (double)c->olon[i];
+        out[1] = (double)c->olat[i];
+        out[2] = 0.0;
+    }
+}
+
+// 21 bits spread to every third bit
+unsigned long long spread3(unsigned long long v)
+{
+    v = (v | (v << 32)) & 0x001f00000000ffffULL;
+    v = (v | (v << 16)) & 0x001f0000ff0000ffULL;
+    v = (v | (v << 8)) & 0x100f00f00f00f00fULL;
+    v = (v | (v << 4)) & 0x10c30c30c30c30c3ULL;
+    v = (v | (v << 2)) & 0x1249249249249249ULL;
+    return v;
+}
+
+// order[k]: the k-th of the n points (xyz[3 i ..]) along a Morton curve over
+// their bounding cube, equal codes in index order (a stable radix sort).
+// Points with a non-finite coordinate sort as if it were the lowest.
+void morton_order(const std::vector<double>& xyz, int n, std::vector<int>& order)
+{
+    double lo[3], ext = 0.0;
+    for (int d = 0; d < 3; ++d) {
+        double a = std::numeric_limits<double>::infinity(), b = -a;
+        for (int i = 0; i < n; ++i) {
+            const double v = xyz[3 * (size_t)i + d];
+            if (std::isfinite(v)) {
+                a = std::min(a, v);
+                b = std::max(b, v);
+            }
+        }
+        lo[d] = (a <= b) ? a : 0.0;
+        if (a <= b)
+            ext = std::max(ext, b - a);
+    }
+    const double scale = (ext > 0.0 && std::isfinite(ext)) ? 2097151.0 / ext : 0.0;
+    std::vector<unsigned long long> key((size_t)n), key2((size_t)n);
+    std::vector<int> tmp((size_t)n);
+    order.resize((size_t)n);
+    for (int i = 0; i < n; ++i) {
+        unsigned long long code = 0;
+        for (int d = 0; d < 3; ++d) {
+            const double f = (xyz[3 * (size_t)i + d] - lo[d]) * scale;
+            const unsigned long long g = (f >= 0.0) ? (unsigned long long)std::min(f, 2097151.0) : 0ULL;
+            code |= spread3(g) << d;
+        }
+        key[(size_t)i] = code;
+        order[(size_t)i] = i;
+    }
+    for (int shift = 0; shift < 64; shift += 11) {
+        size_t count[2049] = {0};
+        for (int i = 0; i < n; ++i)
+            ++count[((key[(size_t)i] >> shift) & 2047) + 1];
+        bool same = false;
+        for (int b = 0; b < 2048 && !same; ++b)
+            same = count[b + 1] == (size_t)n;
+        if (same)
+            continue;
+        for (int b = 0; b < 2048; ++b)
+            count[b + 1] += count[b];
+        for (int i = 0; i < n; ++i) {
+            const size_t p = count[(key[(size_t)i] >> shift) & 2047]++;
+            key2[p] = key[(size_t)i];
+            tmp[p] = order[(size_t)i];
+        }
+        key.swap(key2);
+        order.swap(tmp);
+    }
+}
 
 // a kd-tree node while the tree is built on the host
 struct BuildNode {
@@ -352,7 +431,70 @@ double elapsed(hipEvent_t a, hipEvent_t b)
     return ms;
 }
 
-int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes)
+// the reference's kd-trees (obs_createkdtrees), for the searches that follow
+// their order: each type's observations inserted in ascending index order,
+// then relabelled in preorder (a left child directly follows its parent)
+int ensure_trees(enkfg_ctx* c)
+{
+    if (c->trees_built)
+        return ENKFG_OK;
+    std::vector<int> rowof((size_t)std::max(c->nobs, 1), -1);
+    for (int r = 0; r < c->nobs; ++r)
+        rowof[(size_t)c->perm[(size_t)r]] = r;
+    std::vector<KdNode> dnodes(c->nsearch);
+    std::vector<int> noderow(c->nsearch);
+    for (size_t t = 0; t < c->tinfo.size(); ++t) {
+        const TypeInfo& ti = c->tinfo[t];
+        std::vector<int> ids(c->perm.begin() + ti.node0, c->perm.begin() + ti.node0 + ti.nnode);
+        std::sort(ids.begin(), ids.end());
+        std::vector<double> xyz(3 * ids.size());
+        for (size_t k = 0; k < ids.size(); ++k)
+            obs_coords(c, ids[k], c->types[t].geographic != 0, &xyz[3 * k]);
+        std::vector<BuildNode> nodes;
+        build_tree(xyz, ti.ndim, ids, nodes);
+        if ((int)nodes.size() != ti.nnode)
+            return fail(c, ENKFG_ERR_ARG, "internal: kd-tree of obstype %d is incomplete", (int)t);
+        for (int v = 0; v < ti.nnode; ++v) {
+            const BuildNode& b = nodes[(size_t)v];
+            if (b.left >= 0 && b.left != v + 1)
+                return fail(c, ENKFG_ERR_ARG, "internal: kd-tree of obstype %d is not in preorder", (int)t);
+            KdNode& d = dnodes[(size_t)ti.node0 + v];
+            d.x = b.x;
+            d.y = b.y;
+            d.z = b.z;
+            d.right = b.right;
+            d.link = (unsigned)(b.parent + 1) | (b.left >= 0 ? 0x80000000u : 0u);
+            noderow[(size_t)ti.node0 + v] = rowof[(size_t)b.obsid];
+        }
+    }
+    HIPCHECK(c, c->d_nodes.reserve(std::max<size_t>(dnodes.size(), 1) * sizeof(KdNode)));
+    HIPCHECK(c, c->d_noderow.reserve(std::max<size_t>(noderow.size(), 1) * sizeof(int)));
+    if (!dnodes.empty()) {
+        HIPCHECK(c, hipMemcpy(c->d_nodes.p, dnodes.data(), dnodes.size() * sizeof(KdNode), hipMemcpyHostToDevice));
+        HIPCHECK(c, hipMemcpy(c->d_noderow.p, noderow.data(), noderow.size() * sizeof(int), hipMemcpyHostToDevice));
+    }
+    c->trees_built = true;
+    return ENKFG_OK;
+}
+
+// the lists filled in the reference's order, their offsets known
+hipError_t fill_ordered(enkfg_ctx* c, bool nlobsmax)
+{
+    return launch_loc_fill(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
+                           c->lists_vis ? c->d_vis.as<unsigned char>() : nullptr, c->d_nodes.as<KdNode>(),
+                           c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), (int)c->types.size(),
+                           c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_offsets.as<long long>(),
+                           c->d_ids.as<int>(), c->d_lc.as<double>(), nlobsmax ? c->d_rawoff.as<long long>() : nullptr,
+                           nlobsmax ? c->d_raw.as<int>() : nullptr, nlobsmax ? c->d_srow.as<int>() : nullptr,
+                           nlobsmax ? c->d_sd2.as<double>() : nullptr);
+}
+
+// The lists of every node.  The box search counts them; it fills them too
+// unless the caller wants the reference's order (ordered), for which the
+// trees are walked.  The trees decide alone where the box search does not
+// apply: NLOBSMAX types, non-finite coordinates, and an observation at
+// exactly the radius (which counting finds).
+int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
 {
     if (!c->obs_set)
         return fail(c, ENKFG_ERR_STATE, "observations not set");
@@ -360,6 +502,7 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes)
     for (const auto& t : c->types)
         if (t.nlobsmax != ENKFG_NLOBSMAX_NONE)
             nlobsmax = true;
+    c->lists_valid = false;
     int r = node_inputs(c, nodes);
     if (r != ENKFG_OK)
         return r;
@@ -367,104 +510,86 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes)
     const long long ncnt = (long long)c->nnode * nt;
     HIPCHECK(c, c->d_counts.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
     HIPCHECK(c, c->d_offsets.reserve((ncnt + 1) * sizeof(long long)));
-    const unsigned char* vis = nodes->visible ? c->d_vis.as<unsigned char>() : nullptr;
-    if (nlobsmax)
-        HIPCHECK(c, c->d_raw.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
-    HIPCHECK(c, hipEventRecord(c->ev[0], c->stream));
+    c->lists_vis = nodes->visible != nullptr;
+    const unsigned char* vis = c->lists_vis ? c->d_vis.as<unsigned char>() : nullptr;
+    HIPCHECK(c, c->d_lflag.reserve(sizeof(int)));
     size_t tmpb = 0;
     HIPCHECK(c, launch_scan_counts(c->stream, nullptr, nullptr, ncnt, nullptr, &tmpb));
     HIPCHECK(c, c->d_scantmp.reserve(tmpb));
     tmpb = c->d_scantmp.bytes;
-    if (!nlobsmax && c->pool_cap > 0) {
-        // one walk into the chunk pool, then the compaction; a pool too
-        // small for these lists falls back to the two walks below
-        HIPCHECK(c, c->d_heads.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
-        HIPCHECK(c, c->d_cids.reserve((size_t)c->pool_cap * kLocChunk * sizeof(int)));
-        HIPCHECK(c, c->d_clc.reserve((size_t)c->pool_cap * kLocChunk * sizeof(double)));
-        HIPCHECK(c, c->d_cnext.reserve((size_t)c->pool_cap * sizeof(int)));
-        HIPCHECK(c, c->d_lflag.reserve(2 * sizeof(int)));
-        HIPCHECK(c, hipMemsetAsync(c->d_lflag.p, 0, 2 * sizeof(int), c->stream));
-        HIPCHECK(c, launch_loc_walk(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
-                                    vis, c->d_nodes.as<KdNode>(), c->d_types.as<TypeInfo>(), nt,
-                                    c->d_status.as<short>(), c->d_counts.as<int>(), c->d_heads.as<int>(),
-                                    c->d_cids.as<int>(), c->d_clc.as<double>(), c->d_cnext.as<int>(),
-                                    c->d_lflag.as<int>(), (int)c->pool_cap, c->d_lflag.as<int>() + 1));
+    HIPCHECK(c, hipEventRecord(c->ev[0], c->stream));
+    bool boxes = c->box_ok && !nlobsmax;
+    long long total = 0;
+    if (boxes) {
+        int tie = 0;
+        HIPCHECK(c, hipMemsetAsync(c->d_lflag.p, 0, sizeof(int), c->stream));
+        HIPCHECK(c, launch_loc_box(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
+                                   vis, c->d_types.as<TypeInfo>(), nt, c->d_boxes.as<LocBox>(), c->d_xyz.as<double>(),
+                                   c->nsearch, c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_counts.as<int>(),
+                                   c->d_lflag.as<int>(), nullptr, nullptr, nullptr));
         HIPCHECK(c, launch_scan_counts(c->stream, c->d_counts.as<int>(), c->d_offsets.as<long long>(), ncnt,
                                        c->d_scantmp.p, &tmpb));
-        long long total = 0;
-        int flags[2] = {0, 0};
         HIPCHECK(c, hipMemcpyAsync(&total, c->d_offsets.as<long long>() + ncnt, sizeof total, hipMemcpyDeviceToHost,
                                    c->stream));
-        HIPCHECK(c, hipMemcpyAsync(flags, c->d_lflag.p, sizeof flags, hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(c, hipMemcpyAsync(&tie, c->d_lflag.p, sizeof tie, hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
-        if (flags[1] == 0) {
-            HIPCHECK(c, c->d_ids.reserve((total + kListPad) * sizeof(int)));
-            HIPCHECK(c, c->d_lc.reserve((total + kListPad) * sizeof(double)));
-            HIPCHECK(c, launch_loc_compact(c->stream, ncnt, nt, c->d_types.as<TypeInfo>(), c->d_obsids.as<int>(),
-                                           c->d_counts.as<int>(), c->d_heads.as<int>(),
-                                           c->d_offsets.as<long long>(), c->d_cids.as<int>(), c->d_clc.as<double>(),
-                                           c->d_cnext.as<int>(), c->d_ids.as<int>(), c->d_lc.as<double>()));
-            HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
-            HIPCHECK(c, hipStreamSynchronize(c->stream));
-            c->timings[0] = elapsed(c->ev[0], c->ev[1]);
-            c->lists_valid = true;
-            return ENKFG_OK;
-        }
+        boxes = tie == 0;
     }
-    HIPCHECK(c, launch_loc_count(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(), vis,
-                                 c->d_nodes.as<KdNode>(), c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(),
-                                 c->d_counts.as<int>(), nlobsmax ? c->d_raw.as<int>() : nullptr));
-    if (nlobsmax) {
-        // NLOBSMAX types: candidates in visiting order, sorted by distance,
-        // the first NLOBSMAX with status OK kept (observations.c:1899-1908)
-        HIPCHECK(c, c->d_rawoff.reserve((ncnt + 1) * sizeof(long long)));
-        HIPCHECK(c, launch_scan_counts(c->stream, c->d_raw.as<int>(), c->d_rawoff.as<long long>(), ncnt,
+    if (!boxes || ordered) {
+        r = ensure_trees(c);
+        if (r != ENKFG_OK)
+            return r;
+    }
+    if (!boxes) {
+        if (nlobsmax)
+            HIPCHECK(c, c->d_raw.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
+        HIPCHECK(c, launch_loc_count(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(),
+                                     c->d_glob.as<unsigned char>(), vis, c->d_nodes.as<KdNode>(),
+                                     c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(),
+                                     c->d_counts.as<int>(), nlobsmax ? c->d_raw.as<int>() : nullptr));
+        if (nlobsmax) {
+            // NLOBSMAX types: candidates in visiting order, sorted by distance,
+            // the first NLOBSMAX with status OK kept (observations.c:1899-1908)
+            HIPCHECK(c, c->d_rawoff.reserve((ncnt + 1) * sizeof(long long)));
+            HIPCHECK(c, launch_scan_counts(c->stream, c->d_raw.as<int>(), c->d_rawoff.as<long long>(), ncnt,
+                                           c->d_scantmp.p, &tmpb));
+            long long nraw = 0;
+            HIPCHECK(c, hipMemcpyAsync(&nraw, c->d_rawoff.as<long long>() + ncnt, sizeof nraw, hipMemcpyDeviceToHost,
+                                       c->stream));
+            HIPCHECK(c, hipStreamSynchronize(c->stream));
+            HIPCHECK(c, c->d_rrow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
+            HIPCHECK(c, c->d_srow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
+            HIPCHECK(c, c->d_rd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
+            HIPCHECK(c, c->d_sd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
+            HIPCHECK(c, launch_loc_nlobsmax(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(),
+                                            c->d_glob.as<unsigned char>(), vis, c->d_nodes.as<KdNode>(),
+                                            c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt,
+                                            c->d_status.as<short>(), c->d_raw.as<int>(), c->d_rawoff.as<long long>(),
+                                            c->d_rrow.as<int>(), c->d_rd2.as<double>(), c->d_srow.as<int>(),
+                                            c->d_sd2.as<double>(), c->d_counts.as<int>()));
+        }
+        HIPCHECK(c, launch_scan_counts(c->stream, c->d_counts.as<int>(), c->d_offsets.as<long long>(), ncnt,
                                        c->d_scantmp.p, &tmpb));
-        long long nraw = 0;
-        HIPCHECK(c, hipMemcpyAsync(&nraw, c->d_rawoff.as<long long>() + ncnt, sizeof nraw, hipMemcpyDeviceToHost,
+        HIPCHECK(c, hipMemcpyAsync(&total, c->d_offsets.as<long long>() + ncnt, sizeof total, hipMemcpyDeviceToHost,
                                    c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
-        HIPCHECK(c, c->d_rrow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
-        HIPCHECK(c, c->d_srow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
-        HIPCHECK(c, c->d_rd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
-        HIPCHECK(c, c->d_sd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
-        HIPCHECK(c, launch_loc_nlobsmax(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(),
-                                        c->d_glob.as<unsigned char>(), vis, c->d_nodes.as<KdNode>(),
-                                        c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(), c->d_raw.as<int>(),
-                                        c->d_rawoff.as<long long>(), c->d_rrow.as<int>(), c->d_rd2.as<double>(),
-                                        c->d_srow.as<int>(), c->d_sd2.as<double>(), c->d_counts.as<int>()));
     }
-    HIPCHECK(c, launch_scan_counts(c->stream, c->d_counts.as<int>(), c->d_offsets.as<long long>(), ncnt,
-                                   c->d_scantmp.p, &tmpb));
-    long long total = 0;
-    HIPCHECK(c, hipMemcpyAsync(&total, c->d_offsets.as<long long>() + ncnt, sizeof total, hipMemcpyDeviceToHost,
-                               c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
     // the Gram kernels read up to kListPad entries past the last list
     HIPCHECK(c, c->d_ids.reserve((total + kListPad) * sizeof(int)));
     HIPCHECK(c, c->d_lc.reserve((total + kListPad) * sizeof(double)));
-    HIPCHECK(c, launch_loc_fill(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(), vis,
-                                c->d_nodes.as<KdNode>(), c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(),
-                                c->d_obsids.as<int>(), c->d_offsets.as<long long>(), c->d_ids.as<int>(),
-                                c->d_lc.as<double>(), nlobsmax ? c->d_rawoff.as<long long>() : nullptr,
-                                nlobsmax ? c->d_raw.as<int>() : nullptr, nlobsmax ? c->d_srow.as<int>() : nullptr,
-                                nlobsmax ? c->d_sd2.as<double>() : nullptr));
+    c->lists_ordered = ordered || !boxes;
+    if (c->lists_ordered)
+        HIPCHECK(c, fill_ordered(c, nlobsmax));
+    else
+        HIPCHECK(c, launch_loc_box(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
+                                   vis, c->d_types.as<TypeInfo>(), nt, c->d_boxes.as<LocBox>(), c->d_xyz.as<double>(),
+                                   c->nsearch, c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_counts.as<int>(),
+                                   c->d_lflag.as<int>(), c->d_offsets.as<long long>(), c->d_ids.as<int>(),
+                                   c->d_lc.as<double>()));
     HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->timings[0] = elapsed(c->ev[0], c->ev[1]);
     c->lists_valid = true;
-    // pool for the next localisation's single walk: the chunks these lists
-    // take, and a margin
-    if (!nlobsmax) {
-        std::vector<int> cnt((size_t)ncnt);
-        if (ncnt > 0)
-            HIPCHECK(c, hipMemcpy(cnt.data(), c->d_counts.p, (size_t)ncnt * sizeof(int), hipMemcpyDeviceToHost));
-        long long need = 0;
-        for (int n : cnt)
-            need += (n + kLocChunk - 1) / kLocChunk;
-        need += need / 64 + 64;
-        c->pool_cap = (need < 0x7fffffffLL) ? need : 0;   // 0: stay with the two walks
-    }
     return ENKFG_OK;
 }
 
@@ -554,7 +679,7 @@ void enkfg_destroy(enkfg_ctx* c)
         (void)hipStreamSynchronize(c->stream2);
     DevBuf* bufs[] = {&c->d_nodes, &c->d_types, &c->d_obsids, &c->d_type, &c->d_status, &c->d_estd, &c->d_sqrtrf,
                       &c->d_perm, &c->d_S, &c->d_s, &c->d_tmp, &c->d_tmp2, &c->d_qxyz, &c->d_glob, &c->d_vis, &c->d_counts, &c->d_offsets,
-                      &c->d_scantmp, &c->d_ids, &c->d_lc, &c->d_heads, &c->d_cids, &c->d_clc, &c->d_cnext, &c->d_lflag,
+                      &c->d_scantmp, &c->d_ids, &c->d_lc, &c->d_lflag, &c->d_noderow, &c->d_xyz, &c->d_boxes,
                       &c->d_raw, &c->d_rawoff, &c->d_rrow, &c->d_rd2,
                       &c->d_srow, &c->d_sd2, &c->d_T, &c->d_w, &c->d_T64, &c->d_w64, &c->d_pnlobs,
                       &c->d_pdfs, &c->d_psrf, &c->d_gram, &c->d_order, &c->d_segord, &c->d_sts, &c->d_err, &c->d_E, &c->d_infl, &c->d_nlev,
@@ -627,9 +752,19 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
     c->oestd.assign(estd, estd + nobs);
     c->kmod.clear();
 
-    // trees (obs_createkdtrees)
-    std::vector<BuildNode> nodes;
+    // Rows: per type the obs that are searched -- those of obs_createkdtrees:
+    // status OK, finite first coordinate (kd_insertnode) -- along a Morton
+    // curve, then every other obs.  64 consecutive rows of a type share a box,
+    // 64 boxes one of the next level.
+    c->trees_built = false;
+    c->obs_set = false;
     std::vector<int> obsids;
+    std::vector<double> coords;   // [row][3]
+    std::vector<LocBox> boxes;
+    std::vector<unsigned char> placed((size_t)nobs, 0);
+    c->perm.clear();
+    c->perm.reserve(nobs);
+    c->box_ok = true;
     c->tinfo.assign(nt, TypeInfo{});
     for (int t = 0; t < nt; ++t) {
         const enkfg_obstype& ot = c->types[t];
@@ -645,72 +780,93 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
                 rmax = ot.locrad[k];   // obstype_getmaxlocrad
         }
         ti.range = rmax;
-        ti.node0 = (int)nodes.size();
+        ti.node0 = (int)c->perm.size();
         ti.obsid0 = (int)obsids.size();
         if (ot.statsonly)
             continue;
-        std::vector<int> ids;
+        std::vector<int> found;       // searched obs, in index order
+        std::vector<double> xyz;
         for (int i = 0; i < nobs; ++i)
-            if (type[i] == t && status[i] == ENKFG_STATUS_OK)
-                ids.push_back(i);
-        std::vector<double> xyz(3 * ids.size());
-        for (size_t k = 0; k < ids.size(); ++k) {
-            const int i = ids[k];
-            if (ot.geographic)
-                ll2xyz((double)lon[i], (double)lat[i], &xyz[3 * k]);
-            else {
-                xyz[3 * k] = (double)lon[i];
-                xyz[3 * k + 1] = (double)lat[i];
-                xyz[3 * k + 2] = 0.0;
+            if (type[i] == t && status[i] == ENKFG_STATUS_OK) {
+                double x[3];
+                obs_coords(c, i, ot.geographic != 0, x);
+                // obs_getglobal lists every OK obs in index order, including
+                // those the tree skips
+                obsids.push_back(i);
+                ti.nids++;
+                if (!std::isfinite(x[0]))
+                    continue;
+                if (!std::isfinite(x[1]) || !std::isfinite(x[2]))
+                    c->box_ok = false;
+                found.push_back(i);
+                xyz.insert(xyz.end(), x, x + 3);
+            }
+        ti.nnode = (int)found.size();
+        ti.searchable = ti.nids > 0 ? 1 : 0;
+        std::vector<int> order;
+        morton_order(xyz, ti.nnode, order);
+        for (int k = 0; k < ti.nnode; ++k) {
+            const int q = order[(size_t)k];
+            c->perm.push_back(found[(size_t)q]);
+            placed[(size_t)found[(size_t)q]] = 1;
+            coords.insert(coords.end(), &xyz[3 * (size_t)q], &xyz[3 * (size_t)q] + 3);
+        }
+        for (int level = 0; level < kBoxLevels; ++level) {
+            ti.box0[level] = (int)boxes.size();
+            const int n = level == 0 ? ti.nnode : ti.nbox[level - 1];
+            ti.nbox[level] = (n + 63) / 64;
+            for (int b = 0; b < ti.nbox[level]; ++b) {
+                const float inf = std::numeric_limits<float>::infinity();
+                LocBox bx;
+                bx.pad0 = bx.pad1 = 0.0f;
+                for (int d = 0; d < 3; ++d) {
+                    bx.lo[d] = inf;
+                    bx.hi[d] = -inf;
+                    for (int k = 64 * b; k < std::min(n, 64 * b + 64); ++k) {
+                        float lo, hi;
+                        if (level == 0) {
+                            const double v = coords[3 * ((size_t)ti.node0 + k) + d];
+                            lo = hi = (float)v;
+                            if ((double)lo > v)
+                                lo = std::nextafterf(lo, -inf);
+                            if ((double)hi < v)
+                                hi = std::nextafterf(hi, inf);
+                        } else {
+                            lo = boxes[(size_t)ti.box0[level - 1] + k].lo[d];
+                            hi = boxes[(size_t)ti.box0[level - 1] + k].hi[d];
+                        }
+                        bx.lo[d] = std::min(bx.lo[d], lo);
+                        bx.hi[d] = std::max(bx.hi[d], hi);
+                    }
+                }
+                boxes.push_back(bx);
             }
         }
-        build_tree(xyz, ti.ndim, ids, nodes);
-        ti.nnode = (int)(nodes.size() - ti.node0);
-        // obs_getglobal lists obsids in index order, including obs the tree
-        // skipped for non-finite coordinates
-        obsids.insert(obsids.end(), ids.begin(), ids.end());
-        ti.nids = (int)ids.size();
-        ti.searchable = ids.empty() ? 0 : 1;
     }
-    // row order: each type's tree in preorder, then every obs not in a tree
+    c->nsearch = c->perm.size();
+    for (int i = 0; i < nobs; ++i)
+        if (!placed[(size_t)i])
+            c->perm.push_back(i);
     {
         std::vector<int> rowof((size_t)nobs, -1);
-        c->perm.clear();
-        c->perm.reserve(nobs);
-        for (const BuildNode& nd : nodes)
-            if (rowof[nd.obsid] < 0) {
-                rowof[nd.obsid] = (int)c->perm.size();
-                c->perm.push_back(nd.obsid);
-            }
-        for (int i = 0; i < nobs; ++i)
-            if (rowof[i] < 0) {
-                rowof[i] = (int)c->perm.size();
-                c->perm.push_back(i);
-            }
+        for (int r = 0; r < nobs; ++r)
+            rowof[(size_t)c->perm[(size_t)r]] = r;
         for (int& id : obsids)
-            id = rowof[id];
+            id = rowof[(size_t)id];
     }
-    // device nodes: the row of node k is k (rows follow the node order); in
-    // preorder a left child directly follows its parent
-    std::vector<KdNode> dnodes(nodes.size());
-    for (int t = 0; t < nt; ++t)
-        for (int v = 0; v < c->tinfo[t].nnode; ++v) {
-            const BuildNode& b = nodes[(size_t)c->tinfo[t].node0 + v];
-            if (b.left >= 0 && b.left != v + 1)
-                return fail(c, ENKFG_ERR_ARG, "internal: kd-tree of obstype %d is not in preorder", t);
-            KdNode& d = dnodes[(size_t)c->tinfo[t].node0 + v];
-            d.x = b.x;
-            d.y = b.y;
-            d.z = b.z;
-            d.right = b.right;
-            d.link = (unsigned)(b.parent + 1) | (b.left >= 0 ? 0x80000000u : 0u);
-        }
     HIPCHECK(c, c->d_perm.reserve(std::max(nobs, 1) * sizeof(int)));
     if (nobs > 0)
         HIPCHECK(c, hipMemcpy(c->d_perm.p, c->perm.data(), nobs * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHECK(c, c->d_nodes.reserve(std::max<size_t>(dnodes.size(), 1) * sizeof(KdNode)));
-    if (!dnodes.empty())
-        HIPCHECK(c, hipMemcpy(c->d_nodes.p, dnodes.data(), dnodes.size() * sizeof(KdNode), hipMemcpyHostToDevice));
+    HIPCHECK(c, c->d_xyz.reserve(std::max<size_t>(3 * c->nsearch, 1) * sizeof(double)));
+    HIPCHECK(c, c->d_boxes.reserve(std::max<size_t>(boxes.size(), 1) * sizeof(LocBox)));
+    if (c->nsearch > 0) {
+        std::vector<double> soa(3 * c->nsearch);   // x, y, z of the rows
+        for (size_t r = 0; r < c->nsearch; ++r)
+            for (int d = 0; d < 3; ++d)
+                soa[d * c->nsearch + r] = coords[3 * r + d];
+        HIPCHECK(c, hipMemcpy(c->d_xyz.p, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIPCHECK(c, hipMemcpy(c->d_boxes.p, boxes.data(), boxes.size() * sizeof(LocBox), hipMemcpyHostToDevice));
+    }
     HIPCHECK(c, c->d_obsids.reserve(std::max<size_t>(obsids.size(), 1) * sizeof(int)));
     if (!obsids.empty())
         HIPCHECK(c, hipMemcpy(c->d_obsids.p, obsids.data(), obsids.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -1030,7 +1186,7 @@ int enkfg_localise(enkfg_ctx* c, const enkfg_nodes* nodes)
 {
     if (check_ctx(c))
         return ENKFG_ERR_ARG;
-    return do_localise(c, nodes);
+    return do_localise(c, nodes, true);
 }
 
 int enkfg_get_local_counts(enkfg_ctx* c, int* counts)
@@ -1066,6 +1222,15 @@ int enkfg_get_localobs(enkfg_ctx* c, int node, int cap, int* ids, double* lc)
     const long long p = o[1] - o[0];
     if (p > cap)
         return fail(c, ENKFG_ERR_ARG, "cap %d < %lld local obs", cap, p);
+    if (p > 0 && !c->lists_ordered) {
+        // the calc's lists are in row order; the caller's in the reference's
+        int r = ensure_trees(c);
+        if (r != ENKFG_OK)
+            return r;
+        HIPCHECK(c, fill_ordered(c, false));
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        c->lists_ordered = true;
+    }
     if (p > 0) {
         if (ids != nullptr) {
             HIPCHECK(c, hipMemcpy(ids, c->d_ids.as<int>() + o[0], p * sizeof(int), hipMemcpyDeviceToHost));
@@ -1084,7 +1249,7 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
         return ENKFG_ERR_ARG;
     if (!c->S_set)
         return fail(c, ENKFG_ERR_STATE, "S not set");
-    int r = do_localise(c, nodes);
+    int r = do_localise(c, nodes, false);
     if (r != ENKFG_OK)
         return r;
     const int m = c->cfg.nmem, md = c->cfg.nmem_dynamic;

@@ -13,9 +13,8 @@ namespace enkfg {
 // is the one obs_createkdtrees builds (sequential insertion,
 // common/kdtree.c:194-274), stored in preorder: the left child of node v is
 // v + 1, the split dimension of a node is its depth modulo ndim (as
-// kd_insertnode assigns it), and a node's global index in the node array is
-// its observation's device row.  Parent links allow a stackless depth-first
-// walk.
+// kd_insertnode assigns it).  Parent links allow a stackless depth-first
+// walk.  The device row of a node's observation is in a table of its own.
 struct alignas(16) KdNode {
     double x, y, z;   // coordinates (z unused for 2D trees)
     int right;        // right child within the type's tree, -1 = none
@@ -23,16 +22,26 @@ struct alignas(16) KdNode {
 };
 static_assert(sizeof(KdNode) == 32, "KdNode layout");
 
+// Bounds of 64 observations (level 0) or of 64 boxes of the level below, in
+// single precision rounded outwards
+struct alignas(16) LocBox {
+    float lo[3], pad0;
+    float hi[3], pad1;
+};
+constexpr int kBoxLevels = 3;
+
 // Per-obstype search parameters (obstype fields of common/obstypes.h)
 struct TypeInfo {
-    int node0;        // first node of this type's tree in the node array
-    int nnode;        // nodes in the tree (== OK obs at build time)
+    int node0;        // first device row of this type's obs, and first node of its tree
+    int nnode;        // obs that are searched (== OK obs at build time), rows node0 ..
     int ndim;         // 3 geographic, 2 otherwise
     int searchable;   // tree present and not stats-only
     int nlocrad;
     int nlobsmax;
     int obsid0;       // first entry of this type in the obsids array
     int nids;         // OK obs of this type at tree build (obs_getglobal list)
+    int box0[kBoxLevels];   // first box of each level in the box array
+    int nbox[kBoxLevels];
     double range;     // obstype_getmaxlocrad()
     double locrad[ENKFG_MAXLOCRAD];
     double locweight[ENKFG_MAXLOCRAD];
@@ -42,28 +51,24 @@ struct TypeInfo {
 
 // localisation (loc_kernels.hip)
 hipError_t launch_loc_count(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                            const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
-                            const short* status, int* counts, int* raw);
+                            const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                            const TypeInfo* types, int ntypes, const short* status, int* counts, int* raw);
 // NLOBSMAX types: candidates (raw counts scanned into rawoff) gathered, sorted
 // by distance and selected; writes the list lengths into counts (rrow and
 // rd2 are overwritten)
 hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                               const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
-                               const short* status, const int* raw, const long long* rawoff, int* rrow, double* rd2,
+                               const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                               const TypeInfo* types, int ntypes, const short* status, const int* raw, const long long* rawoff, int* rrow, double* rd2,
                                int* srow, double* sd2, int* counts);
-// one-walk localisation (loc_kernels.hip): lists appended to a pool of
-// chunks of kLocChunk entries, then compacted into the CSR arrays
-constexpr int kLocChunk = 512;
-hipError_t launch_loc_walk(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                           const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
-                           const short* status, int* counts, int* heads, int* cids, double* clc, int* cnext, int* pool,
-                           int pool_cap, int* overflow);
-hipError_t launch_loc_compact(hipStream_t s, long long nitem, int ntypes, const TypeInfo* types, const int* obsids,
-                              const int* counts, const int* heads, const long long* offsets, const int* cids,
-                              const double* clc, const int* cnext, int* ids, double* lc);
+// the box search: with ids == nullptr counts the lists (and sets *tieflag if an
+// observation lies at exactly a type's radius), else fills them
+hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
+                          const unsigned char* visible, const TypeInfo* types, int ntypes, const LocBox* boxes,
+                          const double* xyz, size_t nrow, const short* status, const int* obsids, int* counts,
+                          int* tieflag, const long long* offsets, int* ids, double* lc);
 hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                           const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
-                           const short* status, const int* obsids, const long long* offsets, int* ids,
+                           const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                           const TypeInfo* types, int ntypes, const short* status, const int* obsids, const long long* offsets, int* ids,
                            double* lc, const long long* rawoff, const int* raw, const int* srow, const double* sd2);
 hipError_t launch_scan_counts(hipStream_t s, const int* counts, long long* offsets, long long n, void* tmp,
                               size_t* tmp_bytes);

@@ -1,22 +1,45 @@
 // loc_kernels.hip -- GPU localisation: for every node of the stride grid, the
-// ordered list of (obs id, taper coefficient) that obs_findlocal
+// list of (obs, taper coefficient) that obs_findlocal
 // (common/observations.c:1837-1927) returns.
 //
-// Each thread walks the per-type kd-trees built on the host by sequential
-// insertion (the trees of obs_createkdtrees).  The walk is the preorder of
-// _kd_findnodeswithinrange (common/kdtree.c:516-540) -- node, then the child
-// on the query's side (left iff dx <= 0), then the other child iff |dx| <
-// range -- done without a stack by following parent links: on the way up, a
-// node is re-examined to decide whether the far child is still to be
-// visited, which depends only on that node and the query.  Lists are
-// therefore identical, element for element, to the reference's, including
-// their order.  Squared distances, tapers and the inclusion test use the
-// reference's operation order in IEEE double with no contraction (the
-// library is compiled with -ffp-contract=off), so the taper bits match too.
+// Two searches give the same lists.
 //
-// Two passes: count (per node and type), exclusive scan, fill.  The obs
-// indices in the trees and in the lists are device rows (rows of S in tree
-// preorder); the host maps them back to observation indices.
+// The box search (loc_box_kernel) is what the calc uses, which needs the
+// lists in no particular order.  Rows (and so S) are sorted along a Morton
+// curve per type; 64 consecutive rows make a leaf, 64 boxes a box of the next
+// level, three levels in all.  One wavefront takes one (node, obstype): a
+// step tests 64 boxes or 64 observations with coalesced loads.  Distances
+// and tapers use the reference's operation order in IEEE double with no
+// contraction, and a box is skipped only when its distance, rounded in the
+// same order, exceeds the radius -- rounding is monotone, so no observation
+// of it can be within the radius -- so the set and the taper bits are the
+// tree search's.
+//
+// The tree search walks the reference's own kd-trees (sequential insertion,
+// obs_createkdtrees) in the preorder of _kd_findnodeswithinrange
+// (common/kdtree.c:516-540) -- node, then the child on the query's side (left
+// iff dx <= 0), then the other child iff |dx| < range -- without a stack by
+// following parent links: on the way up, a node is re-examined to decide
+// whether the far child is still to be visited, which depends only on that
+// node and the query.  Its lists are in the reference's order, element for
+// element: enkfg_localise and enkfg_get_localobs return those.  It also
+// decides what the box search cannot: an observation at exactly the radius is
+// in the list only if no split on its path is pruned, non-finite coordinates
+// follow the comparisons of the walk, and NLOBSMAX keeps candidates at equal
+// distance in visiting order.
+//
+// What bounds them, on the 51x1500x1800 tile (300,000 nodes, four types,
+// 1.86G entries, 22 GB of lists): the tree walk by the traffic of its node
+// loads beyond L2 and by the depth of the trees (walking and compacting the
+// lists took 100 ms with the observations in random order, 991 ms in
+// enkf_prep order); the box search, counting and filling, by FP64 issue (a
+// leaf's distances twice, the tapers once) at 17.3 ms in either order.  On
+// 200 x 240 cells and 9 nodes it takes 0.14 ms against 13 ms: a walk's
+// dependent loads are one chain per thread, a box search's steps load 64
+// boxes or 256 observations each.
+//
+// The obs indices in the lists are device rows; the host maps them back to
+// observation indices.
 #include "enkfg_internal.h"
 
 namespace enkfg {
@@ -158,6 +181,7 @@ __global__ void __launch_bounds__(64) loc_count_kernel(int nnode, int ni, const 
                                                         const unsigned char* __restrict__ isglobal,
                                                         const unsigned char* __restrict__ visible,
                                                         const KdNode* __restrict__ nodes,
+                                                        const int* __restrict__ noderow,
                                                         const TypeInfo* __restrict__ types, int ntypes,
                                                         const short* __restrict__ status, int* __restrict__ counts,
                                                         int* __restrict__ raw)
@@ -177,7 +201,7 @@ __global__ void __launch_bounds__(64) loc_count_kernel(int nnode, int ni, const 
             range_walk(nodes + ti.node0, ti.ndim, q, ti.range, [&](int, double) { nraw++; });
         } else if (ti.nnode > 0) {
             range_walk(nodes + ti.node0, ti.ndim, q, ti.range, [&](int v, double) {
-                if (status[ti.node0 + v] == kStatusOK)
+                if (status[noderow[ti.node0 + v]] == kStatusOK)
                     n++;
             });
         }
@@ -193,6 +217,7 @@ __global__ void __launch_bounds__(64) loc_rawfill_kernel(int nnode, int ni, cons
                                                          const unsigned char* __restrict__ isglobal,
                                                          const unsigned char* __restrict__ visible,
                                                          const KdNode* __restrict__ nodes,
+                                                         const int* __restrict__ noderow,
                                                          const TypeInfo* __restrict__ types, int ntypes,
                                                          const long long* __restrict__ rawoff, int* __restrict__ rrow,
                                                          double* __restrict__ rd2)
@@ -207,7 +232,7 @@ __global__ void __launch_bounds__(64) loc_rawfill_kernel(int nnode, int ni, cons
     double q[3] = {qxyz[3 * (size_t)node], qxyz[3 * (size_t)node + 1], qxyz[3 * (size_t)node + 2]};
     long long o = rawoff[(size_t)node * ntypes + t];
     range_walk(nodes + ti.node0, ti.ndim, q, ti.range, [&](int v, double distsq) {
-        rrow[o] = ti.node0 + v;
+        rrow[o] = noderow[ti.node0 + v];
         rd2[o] = distsq;
         o++;
     });
@@ -368,10 +393,20 @@ __global__ void __launch_bounds__(256) loc_sort_big_kernel(int nnode, const Type
         counts[item] = cnt;
 }
 
+// Fills the lists in the reference's order (walked in the tree).  Each thread
+// keeps its entries in registers and writes them as runs that end on a
+// multiple of kLocBurst (32 bytes of ids, 64 of tapers): single 4- and 8-byte
+// stores from 64 threads walking different lists leave their cache lines
+// part-written, and such lines are written back to memory several times over
+// (174 against 105 ms per localisation of the 51x1500x1800 tile; runs of 4
+// gave 118 ms, of 16 106 ms).
+constexpr int kLocBurst = 8;
+
 __global__ void __launch_bounds__(64) loc_fill_kernel(int nnode, int ni, const double* __restrict__ qxyz,
                                                        const unsigned char* __restrict__ isglobal,
                                                        const unsigned char* __restrict__ visible,
                                                        const KdNode* __restrict__ nodes,
+                                                       const int* __restrict__ noderow,
                                                        const TypeInfo* __restrict__ types, int ntypes,
                                                        const short* __restrict__ status,
                                                        const int* __restrict__ obsids,
@@ -407,15 +442,261 @@ __global__ void __launch_bounds__(64) loc_fill_kernel(int nnode, int ni, const d
             }
         }
     } else if (ti.nnode > 0) {
+        int bid[kLocBurst];
+        double blc[kLocBurst];
+#pragma unroll
+        for (int b = 0; b < kLocBurst; ++b) {
+            bid[b] = 0;
+            blc[b] = 0.0;
+        }
+        long long first = o;   // entries first .. o - 1 are in the registers, entry e at e % kLocBurst
         range_walk(nodes + ti.node0, ti.ndim, q, ti.range, [&](int v, double distsq) {
-            const int row = ti.node0 + v;   // device row of the node's observation
-            if (status[row] == kStatusOK) {
-                ids[o] = row;
-                lc[o] = calclcoeff(ti, sqrt(distsq));
-                o++;
+            const int row = noderow[ti.node0 + v];   // device row of the node's observation
+            if (status[row] != kStatusOK)
+                return;
+            const double c = calclcoeff(ti, sqrt(distsq));
+            const int nb = (int)(o % kLocBurst);
+#pragma unroll
+            for (int b = 0; b < kLocBurst; ++b) {
+                bid[b] = (b == nb) ? row : bid[b];
+                blc[b] = (b == nb) ? c : blc[b];
+            }
+            ++o;
+            if (nb == kLocBurst - 1) {
+                const long long w = o - kLocBurst;   // a multiple of kLocBurst
+                if (first <= w) {
+                    int4* di = reinterpret_cast<int4*>(ids + w);
+                    double2* dl = reinterpret_cast<double2*>(lc + w);
+#pragma unroll
+                    for (int b = 0; b < kLocBurst; b += 4)
+                        di[b / 4] = make_int4(bid[b], bid[b + 1], bid[b + 2], bid[b + 3]);
+#pragma unroll
+                    for (int b = 0; b < kLocBurst; b += 2)
+                        dl[b / 2] = make_double2(blc[b], blc[b + 1]);
+                } else {   // the list starts inside this run
+#pragma unroll
+                    for (int b = 0; b < kLocBurst; ++b)
+                        if (w + b >= first) {
+                            ids[w + b] = bid[b];
+                            lc[w + b] = blc[b];
+                        }
+                }
+                first = o;
             }
         });
+        const long long w = o - o % kLocBurst;
+#pragma unroll
+        for (int b = 0; b < kLocBurst; ++b)
+            if (w + b >= first && w + b < o) {
+                ids[w + b] = bid[b];
+                lc[w + b] = blc[b];
+            }
     }
+}
+
+// ---------------------------------------------------------------- box search
+//
+// One wavefront per (node, obstype).  FILL == false counts the lists; FILL ==
+// true, given the scanned offsets, writes them: hits are gathered in LDS and
+// written 64 at a time, so that the tapers are computed with every lane busy
+// and the stores are whole runs.  kBoxAhead leaves are loaded together, since
+// a step's loads, from L2 or beyond, are its latency.
+constexpr int kBoxAhead = 4;
+// consecutive blocks (of four items) per XCD run: four 8 x 8 tiles of nodes
+constexpr int kBoxRun = 64;
+
+// Item `it` as (type, node): 64 consecutive items are an 8 x 8 tile of the
+// stride grid and one type, so the wavefronts in flight on an XCD search a
+// compact patch.  ok is false past the grid's edge.
+__device__ inline bool box_item(long long it, int ni, int nj, int ntypes, int& t, int& node)
+{
+    const int ti = (ni + 7) / 8, tj = (nj + 7) / 8;
+    const long long per_type = (long long)ti * tj * 64;
+    if (it >= per_type * ntypes)
+        return false;
+    t = (int)(it / per_type);
+    const long long rem = it - (long long)t * per_type;
+    const int tile = (int)(rem / 64), k = (int)(rem % 64);
+    const int i = (tile % ti) * 8 + k % 8, j = (tile / ti) * 8 + k / 8;
+    if (i >= ni || j >= nj)
+        return false;
+    node = j * ni + i;
+    return true;
+}
+
+template <int ND>
+__device__ inline double box_distsq(const LocBox& b, double q0, double q1, double q2)
+{
+    // the distance of the nearest point of the box, summed as distsq is; the
+    // difference to a face, and 0 inside
+    double s = 0.0;
+    double d = fmax(fmax((double)b.lo[0] - q0, q0 - (double)b.hi[0]), 0.0);
+    s += d * d;
+    d = fmax(fmax((double)b.lo[1] - q1, q1 - (double)b.hi[1]), 0.0);
+    s += d * d;
+    if (ND == 3) {
+        d = fmax(fmax((double)b.lo[2] - q2, q2 - (double)b.hi[2]), 0.0);
+        s += d * d;
+    }
+    return s;
+}
+
+// orders the LDS accesses of one wavefront
+__device__ inline void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int ND, bool FILL>
+__device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ boxes, const double* __restrict__ xyz,
+                                 size_t nrow, const short* __restrict__ status, const double* q, int* __restrict__ ids,
+                                 double* __restrict__ lc, double* sd, int* si, bool& tie)
+{
+    const int lane = threadIdx.x & 63;
+    const double q0 = q[0], q1 = q[1], q2 = ND == 3 ? q[2] : 0.0;
+    const double r2 = ti.range * ti.range;
+    const LocBox* __restrict__ L1 = boxes + ti.box0[0];
+    const LocBox* __restrict__ L2 = boxes + ti.box0[1];
+    const LocBox* __restrict__ L3 = boxes + ti.box0[2];
+    const double* __restrict__ X = xyz;
+    const double* __restrict__ Y = xyz + nrow;
+    const double* __restrict__ Z = xyz + 2 * nrow;
+    const unsigned long long below = (1ULL << lane) - 1ULL;
+    const int row0 = ti.node0, row1 = ti.node0 + ti.nnode;
+    int n = 0;       // entries counted, or written
+    int nbuf = 0;    // entries in LDS
+    for (int c3 = 0; c3 < ti.nbox[2]; c3 += 64) {
+        const int b3 = c3 + lane;
+        unsigned long long h3 =
+            __ballot(b3 < ti.nbox[2] && !(box_distsq<ND>(L3[min(b3, ti.nbox[2] - 1)], q0, q1, q2) > r2));
+        while (h3) {
+            const int p3 = c3 + __builtin_ctzll(h3);
+            h3 &= h3 - 1;
+            const int b2 = p3 * 64 + lane;
+            unsigned long long h2 =
+                __ballot(b2 < ti.nbox[1] && !(box_distsq<ND>(L2[min(b2, ti.nbox[1] - 1)], q0, q1, q2) > r2));
+            while (h2) {
+                const int p2 = p3 * 64 + __builtin_ctzll(h2);
+                h2 &= h2 - 1;
+                const int b1 = p2 * 64 + lane;
+                unsigned long long h1 =
+                    __ballot(b1 < ti.nbox[0] && !(box_distsq<ND>(L1[min(b1, ti.nbox[0] - 1)], q0, q1, q2) > r2));
+                while (h1) {
+                    int row[kBoxAhead];
+                    double x[kBoxAhead], y[kBoxAhead], z[kBoxAhead];
+                    short st[kBoxAhead];
+#pragma unroll
+                    for (int u = 0; u < kBoxAhead; ++u) {
+                        // past the last hit leaf: a row beyond the type's
+                        row[u] = h1 ? row0 + (p2 * 64 + __builtin_ctzll(h1)) * 64 + lane : row1;
+                        h1 = h1 ? (h1 & (h1 - 1)) : 0ULL;
+                        const int r = min(row[u], row1 - 1);
+                        x[u] = X[r];
+                        y[u] = Y[r];
+                        z[u] = ND == 3 ? Z[r] : 0.0;
+                        st[u] = status[r];
+                    }
+#pragma unroll
+                    for (int u = 0; u < kBoxAhead; ++u) {
+                        // kd_findnodeswithinrange's sum, in its order (kdtree.c:529-533)
+                        double distsq = 0.0;
+                        double d = x[u] - q0;
+                        distsq += d * d;
+                        d = y[u] - q1;
+                        distsq += d * d;
+                        if (ND == 3) {
+                            d = z[u] - q2;
+                            distsq += d * d;
+                        }
+                        const bool in = row[u] < row1 && distsq <= r2;
+                        tie |= in && distsq == r2;
+                        const bool ok = in && st[u] == kStatusOK;
+                        const unsigned long long m = __ballot(ok);
+                        if (!FILL) {
+                            n += __popcll(m);
+                        } else if (m) {
+                            if (ok) {
+                                const int pos = nbuf + __popcll(m & below);
+                                sd[pos] = distsq;
+                                si[pos] = row[u];
+                            }
+                            nbuf += __popcll(m);
+                            wave_lds_fence();
+                            if (nbuf >= 64) {
+                                ids[n + lane] = si[lane];
+                                lc[n + lane] = calclcoeff(ti, sqrt(sd[lane]));
+                                n += 64;
+                                nbuf -= 64;
+                                const double td = sd[64 + lane];
+                                const int tr = si[64 + lane];
+                                wave_lds_fence();
+                                sd[lane] = td;
+                                si[lane] = tr;
+                                wave_lds_fence();
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (FILL && lane < nbuf) {
+        ids[n + lane] = si[lane];
+        lc[n + lane] = calclcoeff(ti, sqrt(sd[lane]));
+    }
+    return n;
+}
+
+template <bool FILL>
+__global__ void __launch_bounds__(256) loc_box_kernel(int ni, int nj, const double* __restrict__ qxyz,
+                                                      const unsigned char* __restrict__ isglobal,
+                                                      const unsigned char* __restrict__ visible,
+                                                      const TypeInfo* __restrict__ types, int ntypes,
+                                                      const LocBox* __restrict__ boxes,
+                                                      const double* __restrict__ xyz, size_t nrow,
+                                                      const short* __restrict__ status, const int* __restrict__ obsids,
+                                                      int* __restrict__ counts, const long long* __restrict__ offsets,
+                                                      int* __restrict__ ids, double* __restrict__ lc,
+                                                      int* __restrict__ tieflag)
+{
+    __shared__ double sd[FILL ? 4 * 128 : 1];
+    __shared__ int si[FILL ? 4 * 128 : 1];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const unsigned s = blockIdx.x / 8, x = blockIdx.x % 8;
+    const long long blk = ((long long)(s / kBoxRun) * 8 + x) * kBoxRun + s % kBoxRun;
+    int t, node;
+    if (!box_item(blk * 4 + wave, ni, nj, ntypes, t, node))
+        return;
+    t = __builtin_amdgcn_readfirstlane(t);   // one item per wavefront
+    node = __builtin_amdgcn_readfirstlane(node);
+    const TypeInfo& ti = types[t];
+    const size_t item = (size_t)node * ntypes + t;
+    int n = 0;
+    if (ti.searchable && (visible == nullptr || visible[t])) {
+        const long long o = FILL ? offsets[item] : 0;
+        if (isglobal[node]) {
+            n = ti.nids;   // obs_getglobal: all obs of the type, no status check
+            if (FILL)
+                for (int i = lane; i < n; i += 64) {
+                    ids[o + i] = obsids[ti.obsid0 + i];
+                    lc[o + i] = 1.0;
+                }
+        } else if (ti.nnode > 0) {
+            const double q[3] = {qxyz[3 * (size_t)node], qxyz[3 * (size_t)node + 1], qxyz[3 * (size_t)node + 2]};
+            bool tie = false;
+            double* wsd = FILL ? sd + wave * 128 : nullptr;
+            int* wsi = FILL ? si + wave * 128 : nullptr;
+            int* wid = FILL ? ids + o : nullptr;
+            double* wlc = FILL ? lc + o : nullptr;
+            n = ti.ndim == 3 ? box_search<3, FILL>(ti, boxes, xyz, nrow, status, q, wid, wlc, wsd, wsi, tie)
+                             : box_search<2, FILL>(ti, boxes, xyz, nrow, status, q, wid, wlc, wsd, wsi, tie);
+            if (!FILL && __ballot(tie) && lane == 0)
+                atomicExch(tieflag, 1);
+        }
+    }
+    if (!FILL && lane == 0)
+        counts[item] = n;
 }
 
 // ---- exclusive scan of int counts into long long offsets (n + 1 entries)
@@ -499,155 +780,6 @@ __global__ void __launch_bounds__(kScanThreads) scan_final_kernel(const int* __r
         out[n] = partials[nb];
 }
 
-// ---------------------------------------------------------------- one walk
-//
-// Counting the lists before filling them walks every tree twice.  With the
-// capacity known from an earlier localisation, one walk suffices: a (node,
-// type) thread appends its entries to chunks of kLocChunk taken from a pool
-// by an atomic counter, linked in order (next[chunk]), and records its count
-// and first chunk; after the scan of the counts, loc_compact_kernel copies
-// each list into its place in the CSR arrays.  A walk that runs out of pool
-// raises the overflow flag; the host then redoes the localisation with the
-// two walks.  Types with NLOBSMAX take the two-walk path.
-//
-// Each thread keeps its last kLocBurst entries in registers and writes them
-// as one aligned run (32 bytes of ids, 64 of tapers): single 4- and 8-byte
-// stores from 64 threads walking different lists leave their cache lines
-// part-written, and such lines are written back to memory several times over.
-constexpr int kLocBurst = 8;
-static_assert(kLocChunk % kLocBurst == 0, "bursts must not straddle chunks");
-
-__global__ void __launch_bounds__(64) loc_walk_kernel(int nnode, int ni, const double* __restrict__ qxyz,
-                                                       const unsigned char* __restrict__ isglobal,
-                                                       const unsigned char* __restrict__ visible,
-                                                       const KdNode* __restrict__ nodes,
-                                                       const TypeInfo* __restrict__ types, int ntypes,
-                                                       const short* __restrict__ status, int* __restrict__ counts,
-                                                       int* __restrict__ heads, int* __restrict__ cids,
-                                                       double* __restrict__ clc, int* __restrict__ cnext,
-                                                       int* __restrict__ pool, int pool_cap, int* __restrict__ overflow)
-{
-    int t, node;
-    if (!thread_node(nnode, ni, ntypes, t, node))
-        return;
-    const size_t item = (size_t)node * ntypes + t;
-    double q[3] = {qxyz[3 * (size_t)node], qxyz[3 * (size_t)node + 1], qxyz[3 * (size_t)node + 2]};
-    const bool glob = isglobal[node] != 0;
-    const TypeInfo& ti = types[t];
-    int n = 0;
-    int head = -1;
-    if (ti.searchable && (visible == nullptr || visible[t])) {
-        if (glob) {
-            n = ti.nids;   // obs_getglobal: all obs of the type, no status check (written by the compaction)
-            head = -2;
-        } else if (ti.nnode > 0) {
-            int cur = -1, pos = kLocChunk;   // pos: entries of chunk cur, written or in the burst
-            int nb = 0;                      // entries in the burst
-            int bid[kLocBurst];
-            double blc[kLocBurst];
-#pragma unroll
-            for (int b = 0; b < kLocBurst; ++b) {
-                bid[b] = 0;
-                blc[b] = 0.0;
-            }
-            bool full = false;
-            range_walk(nodes + ti.node0, ti.ndim, q, ti.range, [&](int v, double distsq) {
-                const int row = ti.node0 + v;   // device row of the node's observation
-                if (status[row] != kStatusOK)
-                    return;
-                n++;
-                if (pos == kLocChunk) {   // the burst is empty here (chunks hold whole bursts)
-                    if (full)
-                        return;
-                    const int nc = atomicAdd(pool, 1);
-                    if (nc >= pool_cap) {
-                        full = true;
-                        return;
-                    }
-                    if (cur >= 0)
-                        cnext[cur] = nc;
-                    else
-                        head = nc;
-                    cur = nc;
-                    pos = 0;
-                }
-                const double c = calclcoeff(ti, sqrt(distsq));
-#pragma unroll
-                for (int b = 0; b < kLocBurst; ++b) {
-                    bid[b] = (b == nb) ? row : bid[b];
-                    blc[b] = (b == nb) ? c : blc[b];
-                }
-                ++nb;
-                ++pos;
-                if (nb == kLocBurst) {
-                    const size_t o = (size_t)cur * kLocChunk + (pos - kLocBurst);   // a multiple of kLocBurst
-                    int4* di = reinterpret_cast<int4*>(cids + o);
-                    double2* dl = reinterpret_cast<double2*>(clc + o);
-#pragma unroll
-                    for (int b = 0; b < kLocBurst; b += 4)
-                        di[b / 4] = make_int4(bid[b], bid[b + 1], bid[b + 2], bid[b + 3]);
-#pragma unroll
-                    for (int b = 0; b < kLocBurst; b += 2)
-                        dl[b / 2] = make_double2(blc[b], blc[b + 1]);
-                    nb = 0;
-                }
-            });
-            if (nb > 0) {
-                const size_t o = (size_t)cur * kLocChunk + (pos - nb);
-#pragma unroll
-                for (int b = 0; b < kLocBurst; ++b)
-                    if (b < nb) {
-                        cids[o + b] = bid[b];
-                        clc[o + b] = blc[b];
-                    }
-            }
-            if (cur >= 0)
-                cnext[cur] = -1;
-            if (full)
-                atomicExch(overflow, 1);
-        }
-    }
-    counts[item] = n;
-    heads[item] = head;
-}
-
-// one wavefront per (node, type): the chunks of a list copied to their
-// place in the CSR arrays (lanes along the chunk: coalesced)
-__global__ void __launch_bounds__(256) loc_compact_kernel(long long nitem, int ntypes,
-                                                           const TypeInfo* __restrict__ types,
-                                                           const int* __restrict__ obsids,
-                                                           const int* __restrict__ counts,
-                                                           const int* __restrict__ heads,
-                                                           const long long* __restrict__ offsets,
-                                                           const int* __restrict__ cids, const double* __restrict__ clc,
-                                                           const int* __restrict__ cnext, int* __restrict__ ids,
-                                                           double* __restrict__ lc)
-{
-    const long long item = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (item >= nitem)
-        return;
-    const int lane = threadIdx.x & 63;
-    const int n = counts[item];
-    const long long o = offsets[item];
-    int cur = heads[item];
-    if (cur == -2) {
-        const TypeInfo& ti = types[item % ntypes];
-        for (int i = lane; i < n; i += 64) {
-            ids[o + i] = obsids[ti.obsid0 + i];
-            lc[o + i] = 1.0;
-        }
-        return;
-    }
-    for (int k0 = 0; k0 < n && cur >= 0; k0 += kLocChunk) {
-        const int len = min(kLocChunk, n - k0);
-        for (int i = lane; i < len; i += 64) {
-            ids[o + k0 + i] = cids[(size_t)cur * kLocChunk + i];
-            lc[o + k0 + i] = clc[(size_t)cur * kLocChunk + i];
-        }
-        cur = cnext[cur];
-    }
-}
-
 // grid of the walk kernels: one 64-thread block per 8 x 8 tile and obstype
 // (thread_node), rounded up to a multiple of 8 runs
 inline dim3 walk_grid(int ni, int nj, int ntypes)
@@ -659,19 +791,21 @@ inline dim3 walk_grid(int ni, int nj, int ntypes)
 }  // namespace
 
 hipError_t launch_loc_count(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                            const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
+                            const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                            const TypeInfo* types, int ntypes,
                             const short* status, int* counts, int* raw)
 {
     const long long nt = (long long)ni * nj * ntypes;
     if (nt <= 0)
         return hipSuccess;
     hipLaunchKernelGGL(loc_count_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
-                       visible, nodes, types, ntypes, status, counts, raw);
+                       visible, nodes, noderow, types, ntypes, status, counts, raw);
     return hipGetLastError();
 }
 
 hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                               const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
+                               const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                            const TypeInfo* types, int ntypes,
                                const short* status, const int* raw, const long long* rawoff, int* rrow, double* rd2,
                                int* srow, double* sd2, int* counts)
 {
@@ -681,7 +815,7 @@ hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz
     if (nt > 0x7fffffffLL)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(loc_rawfill_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
-                       visible, nodes, types, ntypes, rawoff, rrow, rd2);
+                       visible, nodes, noderow, types, ntypes, rawoff, rrow, rd2);
     hipLaunchKernelGGL(loc_sort_kernel, dim3((unsigned)nt), dim3(256), 0, s, ni * nj, types, ntypes, status, raw,
                        rawoff, rrow, rd2, srow, sd2, counts);
     hipLaunchKernelGGL(loc_sort_big_kernel, dim3((unsigned)nt), dim3(256), 0, s, ni * nj, types, ntypes, status, raw,
@@ -690,7 +824,8 @@ hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz
 }
 
 hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                           const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
+                           const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                            const TypeInfo* types, int ntypes,
                            const short* status, const int* obsids, const long long* offsets, int* ids, double* lc,
                            const long long* rawoff, const int* raw, const int* srow, const double* sd2)
 {
@@ -698,7 +833,7 @@ hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, co
     if (nt <= 0)
         return hipSuccess;
     hipLaunchKernelGGL(loc_fill_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
-                       visible, nodes, types, ntypes, status, obsids, offsets, ids, lc, rawoff, raw, srow, sd2);
+                       visible, nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, rawoff, raw, srow, sd2);
     return hipGetLastError();
 }
 
@@ -728,28 +863,24 @@ hipError_t launch_scan_counts(hipStream_t s, const int* counts, long long* offse
     return hipGetLastError();
 }
 
-hipError_t launch_loc_walk(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
-                           const unsigned char* visible, const KdNode* nodes, const TypeInfo* types, int ntypes,
-                           const short* status, int* counts, int* heads, int* cids, double* clc, int* cnext, int* pool,
-                           int pool_cap, int* overflow)
+hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
+                          const unsigned char* visible, const TypeInfo* types, int ntypes, const LocBox* boxes,
+                          const double* xyz, size_t nrow, const short* status, const int* obsids, int* counts,
+                          int* tieflag, const long long* offsets, int* ids, double* lc)
 {
-    const long long nt = (long long)ni * nj * ntypes;
-    if (nt <= 0)
+    if ((long long)ni * nj * ntypes <= 0)
         return hipSuccess;
-    hipLaunchKernelGGL(loc_walk_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
-                       visible, nodes, types, ntypes, status, counts, heads, cids, clc, cnext, pool, pool_cap,
-                       overflow);
-    return hipGetLastError();
-}
-
-hipError_t launch_loc_compact(hipStream_t s, long long nitem, int ntypes, const TypeInfo* types, const int* obsids,
-                              const int* counts, const int* heads, const long long* offsets, const int* cids,
-                              const double* clc, const int* cnext, int* ids, double* lc)
-{
-    if (nitem <= 0)
-        return hipSuccess;
-    hipLaunchKernelGGL(loc_compact_kernel, dim3((unsigned)((nitem + 3) / 4)), dim3(256), 0, s, nitem, ntypes, types,
-                       obsids, counts, heads, offsets, cids, clc, cnext, ids, lc);
+    const long long blocks = (long long)((ni + 7) / 8) * ((nj + 7) / 8) * 16 * ntypes;
+    const long long round = 8LL * kBoxRun;
+    const long long grid = round * ((blocks + round - 1) / round);
+    if (grid > 0x7fffffffLL)
+        return hipErrorInvalidValue;
+    if (ids == nullptr)
+        hipLaunchKernelGGL(loc_box_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, ni, nj, qxyz, isglobal,
+                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, counts, offsets, ids, lc, tieflag);
+    else
+        hipLaunchKernelGGL(loc_box_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, ni, nj, qxyz, isglobal,
+                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, counts, offsets, ids, lc, tieflag);
     return hipGetLastError();
 }
 

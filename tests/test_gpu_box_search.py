@@ -1,0 +1,89 @@
+"""The calc's localisation (box search over Morton-ordered rows) against the
+oracle's tree search, through the C ABI: the counts per type, the lists in
+the reference's order after the calc (enkfg_get_localobs walks the trees for
+it), and T and w of the calc, which used the box search's lists.
+
+Sizes sit at the edges of the boxes (64 rows a leaf, 64 boxes a level).  The
+integer grids put many observations at exactly the radius (3-4-5 triples),
+where the tree search alone decides; a non-finite latitude does too.
+"""
+import numpy as np
+import pytest
+
+import enkfg
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def run_case(types, typ, lon, lat, status, status_search, node_lon, node_lat, geographic, m=20, seed=0):
+    rng = np.random.default_rng(seed)
+    n = len(typ)
+    estd = np.full(n, 0.5, np.float32)
+    HA = rng.standard_normal((m, n)).astype(np.float32)
+    innov = rng.standard_normal(n)
+    ob = O.OracleObs(types, typ, lon, lat, estd, status=status_search, status_at_build=status)
+    S, s = O.standardise(m, ob, HA, innov)
+    ref = O.calc_transforms(1, 1, m, m, 1.0, ob, S, s, node_lon.ravel(), node_lat.ravel(), geographic=geographic)
+    E = enkfg.Engine(m, keep_fp64=True)
+    E.set_obstypes(types)
+    E.set_obs(typ, status, lon, lat, estd)
+    E.set_S(HA, innov, standardised=False)
+    E.set_obs_status(status_search)
+    for again in range(2):
+        E.calc_transforms(node_lon, node_lat, geographic=geographic)
+        T, w, T64, w64 = E.transforms(fp64=True)
+        pn, _, _ = E.diag()
+        assert np.array_equal(pn, ref["pnlobs"])
+        assert E.stats() == ref["stats"]
+        # sums over the local obs in another order: p m additions of 1 / eps
+        for a, b in ((T64, ref["T64"]), (w64, ref["w64"])):
+            assert np.abs(a - b).max() <= 1e-10 * max(np.abs(b).max(), 1e-300)
+        lists = [E.localobs(k, n) for k in range(node_lon.size)] if again == 0 else lists
+    for k, (lo, la) in enumerate(zip(node_lon.ravel(), node_lat.ravel())):
+        ids, lc = ob.findlocal(lo, la, geographic)
+        assert np.array_equal(lists[k][0][:len(ids)], ids) and np.array_equal(lists[k][1][:len(ids)], lc)
+    E.close()
+    return ref["stats"]["nlobs_sum"]
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 4096, 4097, 20000])
+def test_box_search_sizes(n):
+    """n observations of the first type (random, clustered in profiles at the
+    same position), a few of a second with two radii, some not OK, some marked
+    bad after set_obs; nodes inside and outside the observations' bounds, one
+    without coordinates."""
+    print("case box search n=%d" % n, flush=True)
+    rng = np.random.default_rng(n)
+    n2 = 130
+    lon = np.concatenate([rng.uniform(178, 186, n), np.repeat(rng.uniform(178, 186, 13), 10)]).astype(np.float32)
+    lat = np.concatenate([rng.uniform(-3, 4, n), np.repeat(rng.uniform(-3, 4, 13), 10)]).astype(np.float32)
+    typ = np.concatenate([np.zeros(n, np.int16), np.full(n2, 1, np.int16)])
+    o = rng.permutation(n + n2)
+    lon, lat, typ = lon[o], lat[o], typ[o]
+    status = (rng.random(n + n2) < 0.1).astype(np.int16)
+    status2 = np.where(rng.random(n + n2) < 0.1, 5, status).astype(np.int16)
+    types = [dict(locrad=[150.0]), dict(locrad=[90.0, 310.5], locweight=[1.0, 2.0])]
+    nlon, nlat = np.meshgrid(np.linspace(176.0, 188.0, 11), np.linspace(-6.0, 7.0, 5))
+    nlon[0, 3] = np.nan
+    assert run_case(types, typ, lon, lat, status, status2, nlon, nlat, 1) > 0
+
+
+@pytest.mark.parametrize("bad", [False, True])
+def test_box_search_ties_and_nonfinite(bad):
+    """An integer grid in plain coordinates and radius 5: observations at
+    exactly the radius; with `bad`, also observations without a latitude."""
+    print("case box search ties bad=%d" % bad, flush=True)
+    rng = np.random.default_rng(4)
+    x, y = np.meshgrid(np.arange(40), np.arange(30))
+    lon, lat = x.ravel().astype(np.float32), y.ravel().astype(np.float32)
+    o = rng.permutation(lon.size)
+    lon, lat = lon[o], lat[o]
+    typ = (np.arange(lon.size) % 2).astype(np.int16)
+    if bad:
+        lat[[7, 300]] = np.nan
+        lon[11] = np.nan
+    st = np.zeros(lon.size, np.int16)
+    types = [dict(locrad=[5.0], geographic=0), dict(locrad=[4.5], geographic=0)]
+    nlon, nlat = np.meshgrid(np.arange(1.0, 40.0, 6.0), np.arange(2.0, 30.0, 7.0))
+    assert run_case(types, typ, lon, lat, st, st, nlon, nlat, 0) > 0
