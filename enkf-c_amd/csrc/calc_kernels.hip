@@ -7,8 +7,8 @@
 //
 //   gram   (MFMA FP64)  G0 = S^T S and S^T s, streamed from the gathered
 //                       FP32 rows of S, tapered in FP64 on their way to LDS;
-//   factor (LDS/VGPR)   for ETKF with m > 96 (m <= 96, and DEnKF and EnOI:
-//                       factor_wave.hip), M = I + G0 inverted by in-register
+//   factor (LDS/VGPR)   for ETKF with m > 96 (m <= 96: factor_etkf.hip; DEnKF
+//                       and EnOI: factor_tile.hip), M = I + G0 inverted by in-register
 //                       Gauss-Jordan, then
 //                         T = M^-1/2                (= I - (M+M^1/2)^-1 S^T S)
 //                         w = M^-1 S^T s,  dfs = tr(M^-1 G0) (= tr(G S)),
@@ -22,7 +22,7 @@
 // The identities used are those of the User Guide (doc/enkf-userguide.tex:
 // 440-451, 490-522); the per-type diagnostics, which re-solve the analysis
 // with only the obs of one type as the USE_MPIQUEUE build does
-// (transforms.c:853-879), are factor_wave.hip's factor_trace_kernel for
+// (transforms.c:853-879), are factor_tile.hip's factor_trace_kernel for
 // every scheme.
 #include <algorithm>
 
@@ -183,22 +183,14 @@ __device__ __attribute__((always_inline)) inline void item_wave(const CalcArgs& 
     }
     // the copies of the chunks past the end land before the wave ends
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // outputs in the factor kernel's register-block layout, both triangles
-    // (accumulator register i of lane l holds D[4 i + l / 16][l % 16])
-    double* gout = a.gram + (size_t)b * MP * MP;
+    // the accumulators as they stand (register i of lane l holds
+    // D[4 i + l / 16][l % 16])
+    double* gout = a.gram + (size_t)b * gram_size(MT) + lane;
 #pragma unroll
-    for (int t = 0; t < NTG; ++t) {
-        const int f = G + NG * t;
-        const int I = tri_I(MT, f), J = tri_J(MT, f);
+    for (int t = 0; t < NTG; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 16 * I + 4 * i + kq;
-            const int cc = 16 * J + col;
-            gout[gram_index<MT>(r, cc)] = acc[t][i];
-            if (I != J)
-                gout[gram_index<MT>(cc, r)] = acc[t][i];
-        }
-    }
+        for (int i = 0; i < 4; ++i)
+            gout[(G + NG * t) * 256 + 64 * i] = acc[t][i];
     if (G == 0) {
         double* stsout = a.sts + (size_t)b * MP;
 #pragma unroll
@@ -441,7 +433,6 @@ template <int B>
 __device__ inline double load_gram(const CalcArgs& a, int bnode, int seg, double diag, double (&x)[B][B], FactorShared<B>& sh)
 {
     const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
-    const int mp = 16 * ((a.m + 15) / 16);
     const int m = a.m;
     double tr = 0.0;
 #pragma unroll
@@ -456,7 +447,7 @@ __device__ inline double load_gram(const CalcArgs& a, int bnode, int seg, double
         const int cnt = a.pertype ? a.counts[(size_t)node * a.ntypes + s] : 1;
         if (cnt == 0)
             continue;
-        const double* g = a.gram + ((size_t)bnode * a.nseg + s) * mp * mp;
+        const double* g = a.gram + ((size_t)bnode * a.nseg + s) * gram_size(B);
 #pragma unroll
         for (int r = 0; r < B; ++r) {
             const int i = ti * B + r;
@@ -464,7 +455,7 @@ __device__ inline double load_gram(const CalcArgs& a, int bnode, int seg, double
             for (int c = 0; c < B; ++c) {
                 const int j = tj * B + c;
                 if (i < m && j < m)
-                    x[r][c] += g[gram_index<B>(i, j)];
+                    x[r][c] += g[gram_at(B, i, j)];
             }
         }
     }
@@ -490,7 +481,6 @@ template <int B>
 __device__ inline double dot_gram(const CalcArgs& a, int bnode, int seg, const double (&x)[B][B], FactorShared<B>& sh)
 {
     const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
-    const int mp = 16 * ((a.m + 15) / 16);
     const int m = a.m;
     double acc = 0.0;
     for (int s = 0; s < a.nseg; ++s) {
@@ -500,7 +490,7 @@ __device__ inline double dot_gram(const CalcArgs& a, int bnode, int seg, const d
         const int cnt = a.pertype ? a.counts[(size_t)node * a.ntypes + s] : 1;
         if (cnt == 0)
             continue;
-        const double* g = a.gram + ((size_t)bnode * a.nseg + s) * mp * mp;
+        const double* g = a.gram + ((size_t)bnode * a.nseg + s) * gram_size(B);
 #pragma unroll
         for (int r = 0; r < B; ++r) {
             const int i = ti * B + r;
@@ -508,7 +498,7 @@ __device__ inline double dot_gram(const CalcArgs& a, int bnode, int seg, const d
             for (int c = 0; c < B; ++c) {
                 const int j = tj * B + c;
                 if (i < m && j < m)
-                    acc += x[r][c] * g[gram_index<B>(i, j)];
+                    acc += x[r][c] * g[gram_at(B, i, j)];
             }
         }
     }
@@ -852,7 +842,7 @@ void launch_factor_b(hipStream_t s, const CalcArgs& a)
 hipError_t launch_factor(hipStream_t s, const CalcArgs& a)
 {
     if (factor_wave_supported(a))
-        return launch_factor_wave(s, a);   // DEnKF, EnOI: the symmetric sweep (factor_wave.hip)
+        return launch_factor_wave(s, a);   // DEnKF, EnOI (factor_tile.hip)
     // ETKF: by the symmetric sweep up to m = 96; beyond, the Gauss-Jordan
     // kernel with its iterates in device memory
     if (a.m <= 96)

@@ -1270,11 +1270,14 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
 
     const int mp = 16 * ((m + 15) / 16);
     const int nseg = pertype ? nt : 1;
-    const size_t per_node = (size_t)nseg * mp * mp * sizeof(double);
-    // batches of up to 8 GiB of Gram scratch (two buffers): fewer, larger
-    // launches, each ending on a partly empty GPU less often (on the tile 11
-    // batches instead of 42 with 2 GiB: FP64 calc 663 -> 658 ms)
-    const size_t budget = (size_t)8 << 30;
+    const size_t per_node = (size_t)nseg * gram_size(mp / 16) * sizeof(double);
+    // batches of up to 4 GiB of Gram scratch (two buffers): fewer, larger
+    // launches end on a partly empty GPU less often, but the factor of the
+    // last batch runs alone and a first calc allocates them (51x1500x1800
+    // tile, FP64 / mixed calc: 8 GiB 412 / 198 ms, 4 GiB 412 / 201, 2 GiB
+    // 415 / 218, 1 GiB 422 / 220; a first calc of 540x801 cells 110, 91, 79,
+    // 75 ms)
+    const size_t budget = (size_t)4 << 30;
     int nbatch = (int)std::max<size_t>(1, std::min<size_t>(budget / per_node, (size_t)nn));
     if (nbatch > 65536)
         nbatch = 65536;

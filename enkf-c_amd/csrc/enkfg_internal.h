@@ -106,7 +106,7 @@ struct CalcArgs {
     int ms;                        // row stride of S: m rounded up to a multiple of 4
     int nobs;                      // index of the zero row
     // ids and lc are readable for kListPad entries past the last list
-    double* gram;                  // [nbatch][nseg][mp][mp]
+    double* gram;                  // [nbatch][nseg][gram_size(MT)] (gram_layout.h)
     double* sts;                   // [nbatch][nseg][mp]
     float* T;                      // [nnode][md][m]
     float* w;                      // [nnode][m]
@@ -147,13 +147,13 @@ __host__ __device__ inline size_t etkf_ws_per_node(int m)
 hipError_t launch_gram(hipStream_t s, const CalcArgs& a);
 hipError_t launch_gram_mixed(hipStream_t s, const CalcArgs& a);   // gram_mixed.hip
 hipError_t launch_factor(hipStream_t s, const CalcArgs& a);
-// factor_wave.hip: DEnKF / EnOI with m <= 160 by the symmetric sweep; the
+// factor_tile.hip: DEnKF / EnOI with m <= 160, and the adjoint; the
 // per-type diagnostics of every scheme (factor_trace_kernel, after the
 // node's own factorisation on the same stream)
 bool factor_wave_supported(const CalcArgs& a);
 hipError_t launch_factor_wave(hipStream_t s, const CalcArgs& a);
 hipError_t launch_factor_trace(hipStream_t s, const CalcArgs& a);
-// ETKF with m <= 96 by the symmetric sweep, then the per-type diagnostics
+// ETKF with m <= 96 (factor_etkf.hip), then the per-type diagnostics
 hipError_t launch_factor_etkf(hipStream_t s, const CalcArgs& a);
 
 // update (update_kernels.hip)

@@ -91,14 +91,20 @@ __host__ __device__ constexpr int tri_J(int MT, int f)
     return I + f;
 }
 
-// Position of element (i, j) of an m x m matrix (m <= 16 B) in the Gram
-// scratch: the factor kernel's thread (i / B, j / B) of its 16 x 16 thread
-// grid owns the B x B block starting at (B (i / B), B (j / B)), stored as one
-// contiguous run of B * B doubles per thread.
-template <int B>
-__host__ __device__ constexpr size_t gram_index(int i, int j)
+// The Gram scratch of one (node, segment): the upper-triangle tiles in the
+// order above, each 16 x 16 row-major.  Row-major is the accumulator layout of
+// v_mfma_f64_16x16x4_f64 with lane l's register i at 64 i + l, so the Gram
+// kernel stores and the factor kernels load whole 512-byte runs (and 21
+// tiles instead of 36 for m = 96).
+__host__ __device__ constexpr size_t gram_size(int MT) { return (size_t)tri_count(MT) * 256; }
+
+// position of element (i, j) of the symmetric matrix
+__host__ __device__ constexpr size_t gram_at(int MT, int i, int j)
 {
-    return ((size_t)((i / B) * 16 + (j / B)) * B + (i % B)) * B + (j % B);
+    const int I = i / 16, J = j / 16;
+    if (I > J || (I == J && i > j))
+        return gram_at(MT, j, i);
+    return ((size_t)(I * MT - I * (I - 1) / 2 + (J - I)) * 16 + i % 16) * 16 + j % 16;
 }
 
 }  // namespace enkfg

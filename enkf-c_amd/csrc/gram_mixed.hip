@@ -8,7 +8,7 @@
 // (<= 2^-18 relative), so every term of S^T S carries a relative error of
 // about 2^-17 before the FP32 accumulation.  S^T s accumulates in FP64 from
 // hi + lo.  The result is written in the FP64 Gram layout and the
-// factorisation that follows stays in FP64 (factor_wave.hip).
+// factorisation that follows stays in FP64 (factor_tile.hip).
 //
 // Work items, chunk pipeline and XCD placement are those of the FP64 item
 // Gram kernel (calc_kernels.hip, gram_stage.h, gram_layout.h).
@@ -151,21 +151,12 @@ __device__ __attribute__((always_inline)) inline void mix_item_wave(const CalcAr
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // v_mfma_f32_16x16x16_bf16 result: register i of lane l holds
     // D[4 (l / 16) + i][l % 16]
-    double* gout = a.gram + (size_t)b * MP * MP;
+    double* gout = a.gram + (size_t)b * gram_size(MT) + 64 * kg + col;
 #pragma unroll
-    for (int t = 0; t < NTG; ++t) {
-        const int f = G + NG * t;
-        const int I = tri_I(MT, f), J = tri_J(MT, f);
+    for (int t = 0; t < NTG; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 16 * I + 4 * kg + i;
-            const int cc = 16 * J + col;
-            const double v = (double)acc[t][i];
-            gout[gram_index<MT>(r, cc)] = v;
-            if (I != J)
-                gout[gram_index<MT>(cc, r)] = v;
-        }
-    }
+        for (int i = 0; i < 4; ++i)
+            gout[(G + NG * t) * 256 + 16 * i] = (double)acc[t][i];
     if (G == 0) {
         // the four lanes of a member (kg = 0..3) hold partial sums over
         // their 4 obs of each chunk
