@@ -93,16 +93,20 @@ __global__ void permute_rows_kernel(const T* __restrict__ src, const int* __rest
 // ------------------------------------------------------------------ Gram, independent wavefronts
 //
 // Each wavefront computes one group of upper-triangle 16 x 16 tiles (tiles
-// f = g, g + NG, ... of tri_count(MT); NG = 3 groups of 7 tiles or NG = 2
-// groups of 11 and 10 for m = 96, 4 or 5 groups of the 45 tiles for m = 144:
-// item_groups_lo, chosen per obs-count bucket by the host's autotuner) of
-// one (node, obstype segment), with no workgroup barrier: the wave
-// stages its own chunks of IKC local obs through a private LDS area, so the
-// waves of one segment share nothing but L2 (the other waves' copies of the
-// same rows hit there).  Per chunk: the copies of chunks c+1 and c+2 and the
-// list entries of chunk c+3 are in flight while chunk c feeds the MFMAs.
-// The taper is applied in FP64 as an operand is formed, (double) S * lc, as
-// the reference forms Sloc.
+// f = g, g + NG, ... of tri_count(MT); NG = 1 or 2 for m = 96, 4 or 5 groups
+// of the 45 tiles for m = 144: item_groups_lo, chosen per obs-count bucket
+// by the host's autotuner) of one (node, obstype segment), with no workgroup
+// barrier: the wave stages its own chunks of IKC local obs through a private
+// LDS area.  Per chunk: the copies of chunks c+1 and c+2 and the list
+// entries of chunk c+3 are in flight while chunk c feeds the MFMAs.  The
+// taper is applied in FP64 as an operand is formed, (double) S * lc, as the
+// reference forms Sloc.
+//
+// Bound: the FP64 matrix cores (71.7 TFLOP/s in a large library product on
+// this card).  51x1500x1800 tile, 1.771e13 flop: 47 TFLOP/s with two groups
+// and a chunk's conversions ahead of its MFMAs, 56 with one group and the
+// conversions between them, with the factor kernels of the previous batch
+// running beside (calc 412 -> 379 ms).
 // obs per chunk (kChunk, gram_stage.h): four k-steps.  With
 // register-staged chunks, 16 rather than 8 gave a calc pass on the tile of
 // 888 instead of 904 ms: at 8 the Gram took so many waves per CU that the
@@ -111,7 +115,7 @@ __global__ void permute_rows_kernel(const T* __restrict__ src, const int* __rest
 constexpr int IKC = kChunk;
 // chunk buffers (four measured 712.7 against 679.9 ms: six waves per CU)
 constexpr int IKB = 3;
-static_assert(kListPad >= (IKB + 1) * IKC, "list padding too small for the item Gram pipeline");
+static_assert(kListPad >= (IKB + 2) * IKC, "list padding too small for the item Gram pipeline");
 template <int MT>
 using ItemLds = ChunkLds<MT, IKB>;
 
@@ -152,34 +156,68 @@ __device__ __attribute__((always_inline)) inline void item_wave(const CalcArgs& 
     for (int X = 0; X < MT; ++X)
         sts[X] = 0.0;
 
+    // One k-step (four obs) ahead: while the matrix cores work on the
+    // operands of step s, the lane reads, converts and tapers those of step
+    // s + 1, its instructions interleaved with the MFMAs (in a wave's program
+    // order all conversions of a chunk came first, then 44 MFMAs: 73% of the
+    // matrix cores' time).  The last step of a chunk reads the next chunk's
+    // first rows, whose copies chunk_advance waits for; by then every row of
+    // the chunk itself has been read.
     const int nchunk = (cnt + IKC - 1) / IKC;
     chunk_prologue<MT, IKB>(a, sh, off, cnt);
     int buf = 0;    // c % IKB
     int slot = 0;   // c % (IKB + 1)
+    double frag[MT], sl;
+    auto operands = [&](int c, int b2, int sl2, int s, double (&f)[MT], double& t) {
+        const int r = 4 * s + kq;
+        const double lr = reinterpret_cast<const double*>(&sh.meta[sl2][16])[r];
+        const double sv = reinterpret_cast<const double*>(&sh.sv[b2][0])[r];
+        float raw[MT];
+#pragma unroll
+        for (int X = 0; X < MT; ++X)
+            raw[X] = sh.rows[b2][X][r][col];
+        const double l = c * IKC + r < cnt ? lr : 0.0;
+#pragma unroll
+        for (int X = 0; X < MT; ++X)
+            f[X] = (double)raw[X] * l;
+        t = sv * l;
+    };
+    chunk_advance<MT, IKB>(a, sh, off, cnt, 0, buf, slot);
+    operands(0, 0, 0, 0, frag, sl);
     for (int c = 0; c < nchunk; ++c) {
-        chunk_advance<MT, IKB>(a, sh, off, cnt, c, buf, slot);
-        const double* svc = reinterpret_cast<const double*>(&sh.sv[buf][0]);
-        const double* lcc = reinterpret_cast<const double*>(&sh.meta[slot][16]);
+        const int nbuf = buf == IKB - 1 ? 0 : buf + 1;
+        const int nslot = slot == IKB ? 0 : slot + 1;
 #pragma unroll
         for (int s = 0; s < IKC / 4; ++s) {
-            const int r = 4 * s + kq;
-            const double lr = lcc[r];
-            const double l = c * IKC + r < cnt ? lr : 0.0;
-            double frag[MT];
-#pragma unroll
-            for (int X = 0; X < MT; ++X)
-                frag[X] = (double)sh.rows[buf][X][r][col] * l;
+            double fn[MT], sn;
+            if (s == IKC / 4 - 1) {
+                chunk_fence();
+                chunk_advance<MT, IKB>(a, sh, off, cnt, c + 1, nbuf, nslot);
+                operands(c + 1, nbuf, nslot, 0, fn, sn);
+            } else {
+                operands(c, buf, slot, s + 1, fn, sn);
+            }
             item_tiles<MT, NG, G, 0>(frag, acc);
             if (G == 0) {
-                const double sl = svc[r] * l;
 #pragma unroll
                 for (int X = 0; X < MT; ++X)
                     sts[X] += frag[X] * sl;
             }
+            // the LDS reads, then a conversion or product after each MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, MT + 2, 0);
+#pragma unroll
+            for (int t = 0; t < NTG; ++t) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (4 * MT + 8 + NTG - 1) / NTG, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int X = 0; X < MT; ++X)
+                frag[X] = fn[X];
+            sl = sn;
         }
-        chunk_fence();
-        buf = buf == IKB - 1 ? 0 : buf + 1;
-        slot = slot == IKB ? 0 : slot + 1;
+        buf = nbuf;
+        slot = nslot;
     }
     // the copies of the chunks past the end land before the wave ends
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

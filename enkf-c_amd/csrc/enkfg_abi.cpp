@@ -1383,7 +1383,7 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
 
     // Autotuner: the item Gram kernels run a bucket's segments with one of
     // two tile-group counts (wavefronts) per segment, item_groups_lo(MT) or
-    // one more (2 or 3 for m <= 96, 4 or 5 for m = 144).  The first batch of
+    // one more (1 or 2 for m = 96, 4 or 5 for m = 144).  The first batch of
     // a bucket that is not yet tuned for this precision and holds at least
     // kTuneMin nodes runs both and keeps the faster (both write the same
     // Gram matrices, bit for bit); the choice holds for the engine's life.

@@ -130,8 +130,8 @@ struct CalcArgs {
     // ... and, when set, M^-1 of each batch node ([bnode][mp][mp], mp = 16
     // ceil(m / 16), zero outside m x m) for the adjoint through T
     double* adj_minv;
-    // Gram item kernels (m <= 96): tile groups (wavefronts) per segment, 2 or
-    // 3; any other value takes the kernel's default (3 FP64, 2 mixed)
+    // Gram item kernels: tile groups (wavefronts) per segment, item_groups_lo or
+    // one more; any other value takes the default (one more FP64, lo mixed)
     int tile_groups;
     // ETKF with m > 96: the Denman-Beavers iterates Y, Z and Y^-1 of each batch
     // node in device memory, [bnode][3][B * B][256] doubles (thread-major, so

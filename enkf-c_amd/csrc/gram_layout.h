@@ -16,10 +16,14 @@ __host__ __device__ constexpr int tri_count(int MT) { return MT * (MT + 1) / 2; 
 // The item Gram kernels split a segment's tri_count(MT) tiles into NG groups,
 // one wavefront each; the two candidates per MT are lo and lo + 1, lo chosen
 // so that a group's accumulators and operands fit the 256 registers of a
-// lane (21 tiles: 2 or 3 groups; 28: 3 or 4; 36 and 45: 4 or 5; 55: 5 or 6)
+// lane (m = 96: all 21 tiles in one wavefront, 244 registers, so that each
+// observation is read and converted once: FP64 calc on the 51x1500x1800 tile
+// 379 ms against 412 for two groups of unpipelined k-steps; 28 tiles: 3 or 4
+// groups; 36 and 45: 4 or 5; 55: 5 or 6).  Up to m = 64 a segment has ten
+// tiles or fewer and two wavefronts are kept, for launches of few nodes.
 __host__ __device__ constexpr int item_groups_lo(int MT)
 {
-    return MT <= 6 ? 2 : (MT == 7 ? 3 : (MT <= 9 ? 4 : 5));
+    return MT <= 4 ? 2 : (MT <= 6 ? 1 : (MT == 7 ? 3 : (MT <= 9 ? 4 : 5)));
 }
 
 // The items (segment, tile group) of the item Gram kernels are dealt to the 8
