@@ -7,12 +7,13 @@
 // is taken as hi_a hi_b + hi_a lo_b + lo_a hi_b, which leaves out lo_a lo_b
 // (<= 2^-18 relative), so every term of S^T S carries a relative error of
 // about 2^-17 before the FP32 accumulation.  S^T s accumulates in FP64 from
-// hi + lo.  The result is written in the FP64 Gram layout and the
+// x.  The result is written in the FP64 Gram layout and the
 // factorisation that follows stays in FP64 (factor_tile.hip).
 //
 // Work items, chunk pipeline and XCD placement are those of the FP64 item
 // Gram kernel (calc_kernels.hip, gram_stage.h, gram_layout.h).
 #include <algorithm>
+#include <type_traits>
 
 #include "enkfg_internal.h"
 #include "gram_layout.h"
@@ -23,31 +24,32 @@ namespace enkfg {
 namespace {
 
 typedef float flt4 __attribute__((__vector_size__(4 * sizeof(float))));
-typedef __bf16 bf16x4 __attribute__((__vector_size__(4 * sizeof(__bf16))));
 
 // ------------------------------------------------------------------ one wavefront per work item
 //
 // For m <= 160: independent wavefronts, no workgroup barrier.  A wavefront
 // computes one of NG groups of the tri_count(MT) tiles (f = g, g + NG, ...;
-// NG = 2: 11 and 10 tiles for m = 96, NG = 3: 7 each, FP32 accumulators;
+// NG = 1 or 2 for m = 96: all 21 tiles, or 11 and 10, FP32 accumulators;
 // NG is chosen per obs-count bucket by the host's autotuner) of one (node,
 // obstype segment).  The segment's list entries and S rows are copied into
 // the wave's private LDS area in chunks of kChunk = 16 local obs, MKB chunks
 // deep, with no VGPRs held for data in flight (gram_stage.h, the same
-// pipeline as the FP64 item kernel; the other waves of a segment find the
-// rows in L2).  A chunk is one K = 16 step of v_mfma_f32_16x16x16_bf16: lane
-// (col, kg) forms its operand of block X -- obs 4 kg .. 4 kg + 3 of member
-// 16 X + col -- from four FP32 values of the block-major rows, x = S *
-// (float) lc, split into BF16 hi = bf16(x) and lo = bf16(x - hi) (the split
-// carries about 2^-17 relative error); each element is converted once per
-// wave.  S^T s is summed in FP32 over a chunk and in FP64 over chunks.
-// Against the earlier kernel, which gathered one chunk ahead into registers
-// and staged BF16 planes in LDS, the results are the same bit for bit.
+// pipeline as the FP64 item kernel).  Two chunks make one K = 32 step of
+// v_mfma_f32_16x16x32_bf16 (twice the rate of the K = 16 form on this card):
+// lane (col, kg) forms its operand of block X -- obs 4 kg .. 4 kg + 3 of
+// either chunk, member 16 X + col -- from FP32 values of the block-major rows,
+// x = S * (float) lc, split into BF16 hi = bf16(x) and lo = bf16(x - hi) (the
+// split carries about 2^-17 relative error); each element is converted once
+// per wave.  S^T s is summed from x in FP32 over four obs and in FP64 beyond.
+// Bound: VALU issue of the split (about 180 instructions a chunk beside 32
+// MFMAs of 16 cycles for m = 96).  51x1500x1800 tile: mixed calc 201 ms with
+// two wavefronts a list and K = 16, 156 with one, 145 with K = 32 and the
+// operands of the next step formed between the MFMAs.
 constexpr int MKB = 3;
-static_assert(kListPad >= (MKB + 1) * kChunk, "list padding too small for the mixed item Gram pipeline");
+static_assert(kListPad >= (MKB + 4) * kChunk, "list padding too small for the mixed item Gram pipeline");
 template <int MT>
 using MixItemLds = ChunkLds<MT, MKB>;
-typedef short sh4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((__vector_size__(8 * sizeof(__bf16))));
 typedef float flt2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 
@@ -57,18 +59,34 @@ constexpr int mix_item_ntile()
     return (tri_count(MT) - G + NG - 1) / NG;
 }
 
-// the tiles f = G + NG t of group G
-template <int MT, int NG, int G, int T>
-__device__ __attribute__((always_inline)) inline void mix_item_tiles(const sh4 (&h)[MT], const sh4 (&l)[MT],
+// the schedule of half a step: the LDS reads, then the conversions between
+// the MFMAs
+template <int MT, int NM>
+__device__ __attribute__((always_inline)) inline void mix_interleave()
+{
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * MT + 8, 0);
+    if constexpr (NM > 0) {
+#pragma unroll
+        for (int t = 0; t < NM; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, (24 * MT + 30 + NM - 1) / NM, 0);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// the tiles f = G + NG t, T0 <= t < T1, of group G
+template <int MT, int NG, int G, int T0, int T1>
+__device__ __attribute__((always_inline)) inline void mix_item_tiles(const bf16x8 (&h)[MT], const bf16x8 (&l)[MT],
                                                                      flt4* acc)
 {
-    if constexpr (G + NG * T < tri_count(MT)) {
-        constexpr int f = G + NG * T;
+    if constexpr (T0 < T1) {
+        constexpr int f = G + NG * T0;
         constexpr int I = tri_I(MT, f), J = tri_J(MT, f);
-        acc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(h[I], h[J], acc[T], 0, 0, 0);
-        acc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(h[I], l[J], acc[T], 0, 0, 0);
-        acc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(l[I], h[J], acc[T], 0, 0, 0);
-        mix_item_tiles<MT, NG, G, T + 1>(h, l, acc);
+        acc[T0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h[I], h[J], acc[T0], 0, 0, 0);
+        acc[T0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h[I], l[J], acc[T0], 0, 0, 0);
+        acc[T0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[I], h[J], acc[T0], 0, 0, 0);
+        mix_item_tiles<MT, NG, G, T0 + 1, T1>(h, l, acc);
     }
 }
 
@@ -79,7 +97,7 @@ __device__ __attribute__((always_inline)) inline void mix_item_wave(const CalcAr
     constexpr int MP = 16 * MT;
     constexpr int NTG = mix_item_ntile<MT, NG, G>();
     const int lane = threadIdx.x & 63;
-    const int kg = lane >> 4;      // which 4 obs of the K = 16 step
+    const int kg = lane >> 4;      // which 4 obs of a chunk
     const int col = lane & 15;
 
     flt4 acc[NTG > 0 ? NTG : 1];
@@ -96,60 +114,82 @@ __device__ __attribute__((always_inline)) inline void mix_item_wave(const CalcAr
     int buf = 0;    // c % MKB
     int slot = 0;   // c % (MKB + 1)
     const int k0 = 4 * kg;
-    for (int c = 0; c < nchunk; ++c) {
-        chunk_advance<MT, MKB>(a, sh, off, cnt, c, buf, slot);
+    // The operands of a K = 32 step: lane l supplies 8 obs of member row
+    // l % 16 of a tile, here 4 (l / 16) .. of chunk c (HALF 0) and of chunk
+    // c + 1 (HALF 1); which obs is which k does not matter as both operands
+    // agree.  Past the list's end rows and tapers are 0.
+    auto form = [&](auto half, int c, bf16x8 (&h)[MT], bf16x8 (&l)[MT]) {
+        constexpr int o = 4 * decltype(half)::value;
         const double* svc = reinterpret_cast<const double*>(&sh.sv[buf][0]);
         const double* lcc = reinterpret_cast<const double*>(&sh.meta[slot][16]);
-        // tapers of the lane's 4 obs (0 past the list's end) and s * lc
+        // tapers of the lane's 4 obs and s * lc
         float lcf[4], slv[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const double lr = lcc[k0 + q];
-            const double l = c * kChunk + k0 + q < cnt ? lr : 0.0;
-            lcf[q] = (float)l;
-            slv[q] = (float)(svc[k0 + q] * l);
+            const double lq = c * kChunk + k0 + q < cnt ? lr : 0.0;
+            lcf[q] = (float)lq;
+            slv[q] = (float)(svc[k0 + q] * lq);
         }
-        // operand of v_mfma_f32_16x16x16_bf16: lane l supplies 4 consecutive
-        // obs (k = 4 (l / 16) ..) of member row l % 16 of a tile
         // (pairs converted together: v_cvt_pk_bf16_f32)
-        sh4 h[MT], l[MT];
 #pragma unroll
         for (int X = 0; X < MT; ++X) {
-            flt2v x[2], r[2];
-            bf16x2v hp[2], lp[2];
+            float t = 0.0f;
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
-                x[p][0] = sh.rows[buf][X][k0 + 2 * p][col] * lcf[2 * p];
-                x[p][1] = sh.rows[buf][X][k0 + 2 * p + 1][col] * lcf[2 * p + 1];
-                hp[p] = __builtin_convertvector(x[p], bf16x2v);
-                r[p] = x[p] - __builtin_convertvector(hp[p], flt2v);
-                lp[p] = __builtin_convertvector(r[p], bf16x2v);
+                flt2v x;
+                x[0] = sh.rows[buf][X][k0 + 2 * p][col] * lcf[2 * p];
+                x[1] = sh.rows[buf][X][k0 + 2 * p + 1][col] * lcf[2 * p + 1];
+                const bf16x2v hp = __builtin_convertvector(x, bf16x2v);
+                const flt2v r = x - __builtin_convertvector(hp, flt2v);
+                const bf16x2v lp = __builtin_convertvector(r, bf16x2v);
+                h[X][o + 2 * p] = hp[0];
+                h[X][o + 2 * p + 1] = hp[1];
+                l[X][o + 2 * p] = lp[0];
+                l[X][o + 2 * p + 1] = lp[1];
+                if (G == 0) {
+                    t = fmaf(x[0], slv[2 * p], t);
+                    t = fmaf(x[1], slv[2 * p + 1], t);
+                }
             }
-            const bf16x4 hb = {hp[0][0], hp[0][1], hp[1][0], hp[1][1]};
-            const bf16x4 lb = {lp[0][0], lp[0][1], lp[1][0], lp[1][1]};
-            h[X] = __builtin_bit_cast(sh4, hb);
-            l[X] = __builtin_bit_cast(sh4, lb);
-        }
-        mix_item_tiles<MT, NG, G, 0>(h, l, acc);
-        if (G == 0) {
-#pragma unroll
-            for (int X = 0; X < MT; ++X) {
-                const bf16x4 hb = __builtin_bit_cast(bf16x4, h[X]);
-                const bf16x4 lb = __builtin_bit_cast(bf16x4, l[X]);
-                float t = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    t = fmaf((float)hb[q] + (float)lb[q], slv[q], t);
+            if (G == 0)
                 sts[X] += (double)t;
-            }
         }
-        chunk_fence();
+    };
+    auto next = [&](int c) {   // chunk c: its copies have landed, later ones are issued
         buf = buf == MKB - 1 ? 0 : buf + 1;
         slot = slot == MKB ? 0 : slot + 1;
+        chunk_fence();
+        chunk_advance<MT, MKB>(a, sh, off, cnt, c, buf, slot);
+    };
+    // operands one step (two chunks) ahead: while the matrix cores work on
+    // this step's tiles, the lane forms the next step's operands, half of
+    // them beside half of the tiles
+    bf16x8 h[MT], l[MT];
+    chunk_advance<MT, MKB>(a, sh, off, cnt, 0, 0, 0);
+    form(std::integral_constant<int, 0>{}, 0, h, l);
+    next(1);
+    form(std::integral_constant<int, 1>{}, 1, h, l);
+    constexpr int TH = (NTG + 1) / 2;
+    for (int c = 0; c < nchunk; c += 2) {
+        bf16x8 hn[MT], ln[MT];
+        next(c + 2);
+        form(std::integral_constant<int, 0>{}, c + 2, hn, ln);
+        mix_item_tiles<MT, NG, G, 0, TH>(h, l, acc);
+        mix_interleave<MT, 3 * TH>();
+        next(c + 3);
+        form(std::integral_constant<int, 1>{}, c + 3, hn, ln);
+        mix_item_tiles<MT, NG, G, TH, NTG>(h, l, acc);
+        mix_interleave<MT, 3 * (NTG - TH)>();
+#pragma unroll
+        for (int X = 0; X < MT; ++X) {
+            h[X] = hn[X];
+            l[X] = ln[X];
+        }
     }
     // the copies of the chunks past the end land before the wave ends
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // v_mfma_f32_16x16x16_bf16 result: register i of lane l holds
+    // v_mfma_f32_16x16x32_bf16 result: register i of lane l holds
     // D[4 (l / 16) + i][l % 16]
     double* gout = a.gram + (size_t)b * gram_size(MT) + 64 * kg + col;
 #pragma unroll
