@@ -13,13 +13,13 @@
 // per-type diagnostics (calc/transforms.c:843-879), which need only
 // tr(M_t^-1) and tr(G_t).
 //
-// M^-1 = V^T diag(D) V from the block elimination, tr(M^-1) = sum_k tr(D_k) +
-// sum_{i<k} <V_ki, D_k V_ki>.  For m = 96 that is 50 tile products for the
-// elimination, 35 for V, 15 for D V, and for the whole inverse 50 more, of
-// four MFMA instructions each, and six 16 x 16 sweeps.  Bound: the FP64 matrix
-// cores (64 cycles an instruction, 26k cycles a trace) and, beside them, the
-// sweeps' chain of 96 dependent pivots; two wavefronts share a SIMD up to
-// m = 96, so that one's sweep runs beside the other's products.  The padding
+// M^-1 = V^T V from the block Cholesky factorisation, tr(M^-1) = |V|^2.  For
+// m = 96 that is 50 tile products for the factor, 56 for V and 56 more for
+// the whole inverse, of four MFMA instructions each, and six 16 x 16 factors.
+// Bound: the FP64 matrix cores (64 cycles an instruction, 27k cycles a trace)
+// and, beside them, the chain of 96 dependent pivots; two wavefronts share a
+// SIMD up to m = 96, so that one's pivots run beside the other's products.
+// The padding
 // (rows m ..) is an identity block, which the elimination leaves intact.
 //
 // Measured against the kernels before it, which kept a matrix in 4 x 4 to 10 x
@@ -36,78 +36,6 @@
 namespace enkfg {
 
 namespace {
-
-constexpr double kDfsMin = 1.0e-6;   // DFS_MIN, calc/transforms.c:32
-
-__device__ inline double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1)
-        v += __shfl_xor(v, o);
-    return v;
-}
-
-// x <- I + the Gram matrices of segments s0 .. s1 - 1 (ONE: s0) of batch node bnode;
-// returns the trace of the Gram matrix
-template <int MT, bool ONE>
-__device__ __attribute__((always_inline)) inline double load_tiles(const CalcArgs& a, int bnode, int node, int s0,
-                                                                   int s1, int lane, tile4* x)
-{
-    constexpr int NT = tri_count(MT);
-    // the first segment's tiles are loaded straight into x, all at once; the
-    // others' kGroup at a time (the loads in flight need registers beside x)
-    constexpr int kGroup = MT <= 7 ? 7 : 4;
-    const double* g = a.gram + ((size_t)bnode * a.nseg + s0) * gram_size(MT) + lane;
-    int s = s0;
-    if (!ONE && a.pertype)
-        while (s < s1 - 1 && a.counts[(size_t)node * a.ntypes + s] == 0)
-            ++s;
-    const double* gs = g + (size_t)(s - s0) * gram_size(MT);
-#pragma unroll
-    for (int f = 0; f < NT; ++f)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            x[f][r] = gs[f * 256 + 64 * r];
-#pragma unroll
-    for (int f = 0; f < NT; ++f)
-        tile_pin(x[f]);
-    __builtin_amdgcn_sched_barrier(0);
-    for (++s; !ONE && s < s1; ++s) {
-        if (a.pertype && a.counts[(size_t)node * a.ntypes + s] == 0)
-            continue;
-        gs = g + (size_t)(s - s0) * gram_size(MT);
-        static_for<0, (NT + kGroup - 1) / kGroup>([&](auto gc) {
-            constexpr int f0 = gc * kGroup;
-            constexpr int n = f0 + kGroup < NT ? kGroup : NT - f0;
-            tile4 t[n];
-#pragma unroll
-            for (int f = 0; f < n; ++f)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    t[f][r] = gs[(f0 + f) * 256 + 64 * r];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int f = 0; f < n; ++f)
-                x[f0 + f] += t[f];
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    }
-    if (!ONE) {
-#pragma unroll
-        for (int f = 0; f < NT; ++f)
-            tile_pin(x[f]);
-    }
-    double tr = 0.0;
-#pragma unroll
-    for (int k = 0; k < MT; ++k)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (4 * r + (lane >> 4) == (lane & 15)) {
-                tr += x[tri_at<MT>(k, k)][r];
-                x[tri_at<MT>(k, k)][r] += 1.0;
-            }
-    return wave_sum(tr);
-}
 
 template <int MT>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves(MT)))) factor_trace_kernel(CalcArgs a)
@@ -153,47 +81,20 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
     tile_invert_factor<MT>(x, lane);
     if (__ballot(bad) && lane == 0)
         atomicExch(a.err, ENKFG_ERR_LINALG);
-    // -tr(M^-1)
+    // tr(M^-1) = |V|^2
     double s = 0.0;
-    static_for<0, MT>([&](auto lc) {
-        constexpr int l = lc;
-        const tile4& d = x[tri_at<MT>(l, l)];
+#pragma unroll
+    for (int f = 0; f < tri_count(MT); ++f)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            s += (4 * r + (lane >> 4) == (lane & 15)) ? d[r] : 0.0;
-        static_for<0, l>([&](auto ic) {
-            constexpr int i = ic;
-            tile4 g = {0.0, 0.0, 0.0, 0.0};
-            tile_mma(g, d, x[tri_at<MT>(i, l)]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                s = fma(g[r], x[tri_at<MT>(i, l)][r], s);
-        });
-    });
-    s = wave_sum(s) + (double)(16 * MT - m);
+            s = fma(x[f][r], x[f][r], s);
+    s = wave_sum(s) - (double)(16 * MT - m);
     if (lane == 0) {
-        const float fd = (float)((double)m + s);
+        const float fd = (float)((double)m - s);
         a.pdfs[o] = fd;
         a.psrf[o] = ((double)fd > kDfsMin) ? (float)(sqrt(trg / (double)fd) - 1.0) : 0.0f;
     }
 }
-
-// a zero tile that the compiler forms only here, in program order: products
-// into it are not taken ahead of the outputs of earlier tiles, for which
-// there are no registers
-__device__ __attribute__((always_inline)) inline tile4 ordered_zero()
-{
-    double z = 0.0;
-    asm volatile("" : "+v"(z)::"memory");
-    return tile4{z, z, z, z};
-}
-
-template <int MT>
-struct TileLds {
-    double b[16 * MT];      // S^T s over the node's segments
-    double g[16 * MT];      // adjoint: dJ/dw of the node
-    double t[16][17];       // a tile, for its transpose
-};
 
 // ADJ: z = M^-1 g and w = M^-1 S^T s per listed node, and M^-1 itself
 template <int MT, bool ADJ>
@@ -276,11 +177,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
     for (int f = 0; f < tri_count(MT); ++f)
         tile_pin(x[f]);
 
-    // -M^-1, tile columns from the last: (M^-1)_ij = V_ji^T D_j + sum_{l>j}
-    // V_li^T (D_l V_lj).  Columns left of j do not need V_lj any more, so
-    // -D_l V_lj takes its place; a tile and its transpose are written as soon
-    // as it is known.  yb[e] = -(M^-1 b) from this lane's rows of column
-    // block e (yg: of g).
+    // M^-1, a tile and its transpose written as soon as it is known; yb[e] =
+    // (M^-1 b) from this lane's rows of column block e (yg: of g)
     const int col = lane & 15, grp = lane >> 4;
     double yb[MT], yg[ADJ ? MT : 1];
     double trx = 0.0;
@@ -294,7 +192,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
     // rows of T (adjoint: of M^-1) to write, in FP32 and FP64
     const int tlim = dotT ? md : 0;
     const int tlim64 = ADJ ? (a.adj_minv != nullptr ? MP : 0) : (dotT && a.T64 != nullptr ? md : 0);
-    auto put = [&](auto ic, auto jc, const tile4& v) {   // tile (I, J) of -M^-1
+    auto put = [&](auto ic, auto jc, const tile4& v) {   // tile (I, J) of M^-1
         constexpr int I = ic, J = jc;
         // the lane's place, opaque in each tile: what is derived from it is
         // formed where it is used, and the tiles are taken one after another,
@@ -309,10 +207,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
             const int e1 = 16 * I + 4 * r + grp, e2 = 16 * J + col;
             if (ADJ) {
                 if (e1 < t64)
-                    a.adj_minv[((size_t)bnode * MP + e1) * MP + e2] = (e1 < m && e2 < m) ? -v[r] : 0.0;
+                    a.adj_minv[((size_t)bnode * MP + e1) * MP + e2] = (e1 < m && e2 < m) ? v[r] : 0.0;
             } else {
                 const double dlt = (e1 == e2) ? 1.0 : 0.0;
-                double t = 0.5 * -v[r] + 0.5 * dlt;
+                double t = 0.5 * v[r] + 0.5 * dlt;
                 t = (t - dlt) * a.alpha + dlt;
                 const size_t o = ((size_t)node * md + e1) * m + e2;
                 if (e1 < t32 && e2 < m)
@@ -338,33 +236,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
             yg[ADJ ? J : 0] = z;
         }
     };
-    static_for<0, MT>([&](auto jr) {
-        constexpr int j = MT - 1 - jr;
-        tile4 jj = x[tri_at<MT>(j, j)];
-        static_for<j + 1, MT>([&](auto lc) {
-            constexpr int l = lc;
-            tile4 g = ordered_zero();
-            tile_mma(g, x[tri_at<MT>(l, l)], x[tri_at<MT>(j, l)]);
-            tile_mma(jj, x[tri_at<MT>(j, l)], g);
-            x[tri_at<MT>(j, l)] = g;
-            tile_pin(x[tri_at<MT>(j, l)]);
-        });
-        tile_pin(jj);
+    tile_inverse<MT>(x, [&](auto ic, auto jc, tile4& v) {
+        constexpr int i = ic, j = jc;
+        put(ic, jc, v);
+        if constexpr (i == j) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            trx += (4 * r + grp == col) ? jj[r] : 0.0;
-        asm volatile("" : "+v"(trx));
-        put(std::integral_constant<int, j>{}, std::integral_constant<int, j>{}, jj);
-        static_for<0, j>([&](auto ic) {
-            constexpr int i = ic;
-            tile4 v = ordered_zero();
-            tile_mma(v, x[tri_at<MT>(i, j)], x[tri_at<MT>(j, j)]);
-            static_for<j + 1, MT>([&](auto lc) {
-                constexpr int l = lc;
-                tile_mma(v, x[tri_at<MT>(i, l)], x[tri_at<MT>(j, l)]);
-            });
-            tile_pin(v);
-            put(std::integral_constant<int, i>{}, std::integral_constant<int, j>{}, v);
+            for (int r = 0; r < 4; ++r)
+                trx += (4 * r + grp == col) ? v[r] : 0.0;
+            asm volatile("" : "+v"(trx));
+        } else {
             __syncthreads();
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -373,17 +253,17 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 v[r] = sh.t[col][4 * r + grp];
-            put(std::integral_constant<int, j>{}, std::integral_constant<int, i>{}, v);
-        });
+            put(jc, ic, v);
+        }
     });
-    trx = wave_sum(trx) + (double)(MP - m);
+    trx = wave_sum(trx) - (double)(MP - m);
     if (!ADJ && lane == 0) {
-        const float fd = (float)((double)m + trx);   // m - tr(M^-1)
+        const float fd = (float)((double)m - trx);   // m - tr(M^-1)
         a.pnlobs[(size_t)nt * a.nnode + node] = p;
         a.pdfs[(size_t)nt * a.nnode + node] = fd;
         a.psrf[(size_t)nt * a.nnode + node] = (float)(sqrt(trg / (double)fd) - 1.0);
     }
-    // w (z) = -(the columns' sums over the four row groups)
+    // w (z): the columns' sums over the four row groups
 #pragma unroll
     for (int k = 0; k < MT; ++k) {
         double y = yb[k];
@@ -395,13 +275,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
             z += __shfl_xor(z, 16);
             z += __shfl_xor(z, 32);
             if (grp == 0 && e < m) {
-                a.adj_w[lk * m + e] = -y;
-                a.adj_z[lk * m + e] = -z;
+                a.adj_w[lk * m + e] = y;
+                a.adj_z[lk * m + e] = z;
             }
         } else if (grp == 0 && e < m) {
-            a.w[(size_t)node * m + e] = (float)-y;
+            a.w[(size_t)node * m + e] = (float)y;
             if (a.w64 != nullptr)
-                a.w64[(size_t)node * m + e] = -y;
+                a.w64[(size_t)node * m + e] = y;
         }
     }
 }
