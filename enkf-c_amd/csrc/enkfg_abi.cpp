@@ -1281,14 +1281,10 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
     int nbatch = (int)std::max<size_t>(1, std::min<size_t>(budget / per_node, (size_t)nn));
     if (nbatch > 65536)
         nbatch = 65536;
-    // ETKF with m > 96 keeps its iterates in device memory (etkf_ws): batches
-    // of at most 1 GiB of it
-    const bool etkf_ws = c->cfg.scheme == ENKFG_SCHEME_ETKF && dotT && m > 96;
-    if (etkf_ws) {
-        const size_t per = etkf_ws_per_node(m) * sizeof(double);
-        nbatch = std::max(1, std::min(nbatch, (int)(((size_t)1 << 30) / per)));
-        HIPCHECK(c, c->d_etkf.reserve((size_t)nbatch * per));
-    }
+    // ETKF keeps its iterates in device memory
+    const bool etkf_ws = c->cfg.scheme == ENKFG_SCHEME_ETKF && dotT;
+    if (etkf_ws)
+        HIPCHECK(c, c->d_etkf.reserve((size_t)etkf_groups(m, nbatch) * etkf_ws_size(m) * sizeof(double)));
     // two scratch buffers: the Gram kernel of batch b + 1 runs while the
     // factor kernel of batch b reads the other one
     const size_t gram_elems = (size_t)nbatch * per_node / sizeof(double);

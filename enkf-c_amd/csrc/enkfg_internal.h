@@ -133,17 +133,17 @@ struct CalcArgs {
     // Gram item kernels: tile groups (wavefronts) per segment, item_groups_lo or
     // one more; any other value takes the default (one more FP64, lo mixed)
     int tile_groups;
-    // ETKF with m > 96: the Denman-Beavers iterates Y, Z and Y^-1 of each batch
-    // node in device memory, [bnode][3][B * B][256] doubles (thread-major, so
-    // each thread's block elements are coalesced)
+    // ETKF: workspace of etkf_groups(m, nbatch) wavefronts, etkf_ws_size(m)
+    // doubles each
     double* etkf_ws;
 };
-// doubles of etkf_ws per batch node
-__host__ __device__ inline size_t etkf_ws_per_node(int m)
+// the upper tiles of three iterates of the Denman-Beavers iteration
+__host__ __device__ inline size_t etkf_ws_size(int m)
 {
-    const size_t B = (size_t)(m + 15) / 16;
-    return 3 * B * B * 256;
+    const size_t MT = (size_t)(m + 15) / 16;
+    return 3 * (MT * (MT + 1) / 2) * 256;
 }
+int etkf_groups(int m, int nbatch);   // factor_etkf.hip
 hipError_t launch_gram(hipStream_t s, const CalcArgs& a);
 hipError_t launch_gram_mixed(hipStream_t s, const CalcArgs& a);   // gram_mixed.hip
 hipError_t launch_factor(hipStream_t s, const CalcArgs& a);
@@ -153,7 +153,7 @@ hipError_t launch_factor(hipStream_t s, const CalcArgs& a);
 bool factor_wave_supported(const CalcArgs& a);
 hipError_t launch_factor_wave(hipStream_t s, const CalcArgs& a);
 hipError_t launch_factor_trace(hipStream_t s, const CalcArgs& a);
-// ETKF with m <= 96 (factor_etkf.hip), then the per-type diagnostics
+// ETKF (factor_etkf.hip), then the per-type diagnostics
 hipError_t launch_factor_etkf(hipStream_t s, const CalcArgs& a);
 
 // update (update_kernels.hip)

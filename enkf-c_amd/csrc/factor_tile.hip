@@ -76,8 +76,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
     tile4 x[tri_count(MT)];
     const double trg = load_tiles<MT, true>(a, bnode, node, t, t + 1, lane, x);
     bool bad = false;
-    double logdet;
-    tile_eliminate<MT>(x, lane, bad, logdet);
+    float log2det;
+    tile_eliminate<MT>(x, lane, bad, log2det);
     tile_invert_factor<MT>(x, lane);
     if (__ballot(bad) && lane == 0)
         atomicExch(a.err, ENKFG_ERR_LINALG);
@@ -167,8 +167,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
     }
     __syncthreads();
     bool bad = false;
-    double logdet;
-    tile_eliminate<MT>(x, lane, bad, logdet);
+    float log2det;
+    tile_eliminate<MT>(x, lane, bad, log2det);
     tile_invert_factor<MT>(x, lane);
     if (__ballot(bad) && lane == 0)
         atomicExch(a.err, ENKFG_ERR_LINALG);
