@@ -37,6 +37,7 @@
 //   The inflation's dependence on the forecast spread involves no
 //   observation.
 #include "enkfg_internal.h"
+#include "tile_matrix.h"
 #include "update_interp.h"
 
 namespace enkfg {
@@ -134,17 +135,25 @@ __global__ void __launch_bounds__(64) adj_cell_kernel(UpdArgs a, const float* __
     }
 }
 
-// one workgroup per listed node of the batch: the node's local obs in
-// parallel; with B (the batch's [bnode][MP][MP]), the term of T as well
-template <int MT>
-__global__ void __launch_bounds__(256) adj_obs_kernel(CalcArgs a, const int* __restrict__ perm,
+// Workgroup (k, y): 16 obs at a time per wavefront of the local obs of listed
+// node k of the batch, wavefront w taking chunks 4 y + w, 4 y + w + 4 gridDim.y,
+// ...; with B (the batch's [bnode][MP][MP]), the term of T as well.
+//
+// S_o B S_o^T is the row sum of (S B) o S with the rows S of 16 obs: S B by
+// FP64 MFMA, obs by members, with B staged in LDS (rows padded by four
+// doubles: the four row groups of an operand read then fall in two disjoint
+// halves of the banks).  One thread per obs with B from memory took 5.5 ms for
+// 441 nodes of 1,500 obs at m = 96.
+template <int MT, bool TERM_T>
+__global__ void __launch_bounds__(256, 2) adj_obs_kernel(CalcArgs a, const int* __restrict__ perm,
                                                       const short* __restrict__ type, const float* __restrict__ estd,
                                                       const double* __restrict__ sqrt_rf,
                                                       const double* __restrict__ B, double* __restrict__ gy,
                                                       double* __restrict__ gR)
 {
-    constexpr int MP = 16 * MT;
+    constexpr int MP = 16 * MT, LB = MP + 4;
     __shared__ double zs[MP], ws[MP];
+    __shared__ double bs[TERM_T ? MP * LB : 1];
     const int k = blockIdx.x;
     if (k >= a.nbatch)
         return;
@@ -155,66 +164,104 @@ __global__ void __launch_bounds__(256) adj_obs_kernel(CalcArgs a, const int* __r
         zs[e] = (e < m) ? a.adj_z[kk * m + e] : 0.0;
         ws[e] = (e < m) ? a.adj_w[kk * m + e] : 0.0;
     }
+    if (TERM_T)
+        for (int q = threadIdx.x; q < MP * MP; q += 256)
+            bs[(q / MP) * LB + q % MP] = B[(size_t)k * MP * MP + q];
     __syncthreads();
-    const double* Bk = B ? B + (size_t)k * MP * MP : nullptr;
     const long long off = a.offsets[(size_t)node * a.ntypes];
-    const long long end = a.offsets[(size_t)(node + 1) * a.ntypes];
+    const int p = (int)(a.offsets[(size_t)(node + 1) * a.ntypes] - off);
     const double sqm = sqrt((double)(m - 1));
-    for (long long q = off + threadIdx.x; q < end; q += 256) {
-        const int row = a.ids[q];
-        const double lc = a.lc[q];
-        const float* Sr = a.S + (long long)row * a.ms;
-        double az = 0.0, aw = 0.0;
-        for (int e = 0; e < m; ++e) {
-            const double sv = (double)Sr[e] * lc;
-            az = fma(sv, zs[e], az);
-            aw = fma(sv, ws[e], aw);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 15, grp = lane >> 4;
+    for (int c = 4 * (int)blockIdx.y + wave; 16 * c < p; c += 4 * (int)gridDim.y) {
+        // B is read from LDS in each pass (held, it would take 288 registers)
+        int bo = 4 * grp * LB + col;
+        asm volatile("" : "+v"(bo));
+        // obs of this lane as an operand (col), and as a result (4 r + grp)
+        const int oc = 16 * c + col;
+        const int rowc = oc < p ? a.ids[off + oc] : a.nobs;   // the zero row past the end
+        const double lcc = oc < p ? a.lc[off + oc] : 0.0;
+        int row[4];
+        double lc[4], az[4], aw[4], qf[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = 16 * c + 4 * r + grp;
+            row[r] = o < p ? a.ids[off + o] : a.nobs;
+            lc[r] = o < p ? a.lc[off + o] : 0.0;
+            az[r] = aw[r] = qf[r] = 0.0;
         }
-        double qf = 0.0;   // S_o B S_o^T, in blocks of 16 members
-        if (Bk != nullptr) {
-#pragma unroll 1
-            for (int ib = 0; ib < MT; ++ib) {
-                double si[16];
+        // operand register r of block K: member 16 K + 4 grp + r of obs col
+        double s[MT][4];
+        if (TERM_T) {
+            const float* Sc = a.S + (long long)rowc * a.ms + 4 * grp;
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
-                    si[u] = (16 * ib + u < m) ? (double)Sr[16 * ib + u] * lc : 0.0;
-#pragma unroll 1
-                for (int jb = 0; jb < MT; ++jb) {
-                    double sj[16];
-#pragma unroll
-                    for (int u = 0; u < 16; ++u)
-                        sj[u] = (16 * jb + u < m) ? (double)Sr[16 * jb + u] * lc : 0.0;
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) {
-                        const double* br = Bk + (size_t)(16 * ib + u) * MP + 16 * jb;
-                        double t = 0.0;
-#pragma unroll
-                        for (int v = 0; v < 16; ++v)
-                            t = fma(br[v], sj[v], t);
-                        qf = fma(si[u], t, qf);
-                    }
-                }
+            for (int K = 0; K < MT; ++K) {
+                const bool in = 16 * K + 4 * grp < a.ms;
+                const float4 v = in ? *reinterpret_cast<const float4*>(Sc + 16 * K) : make_float4(0.f, 0.f, 0.f, 0.f);
+                s[K][0] = (double)v.x * lcc;
+                s[K][1] = (double)v.y * lcc;
+                s[K][2] = (double)v.z * lcc;
+                s[K][3] = (double)v.w * lcc;
             }
         }
-        const double r = a.sv[row] * lc - aw;
-        const int o = perm[row];
-        const double sd = (double)estd[o];
-        const double d = sd * sqrt_rf[type[o]] * sqm;
-        atomicAdd(&gy[row], az * lc / d);
-        atomicAdd(&gR[row], (-az * r + qf) / (sd * sd));
+#pragma unroll
+        for (int J = 0; J < MT; ++J) {
+            const int e = 16 * J + col;
+            tile4 y = {0.0, 0.0, 0.0, 0.0};
+            if (TERM_T) {
+#pragma unroll
+                for (int K = 0; K < MT; ++K)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        y = __builtin_amdgcn_mfma_f64_16x16x4f64(s[K][r], bs[bo + (16 * K + r) * LB + 16 * J], y, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double sv = e < m ? (double)a.S[(long long)row[r] * a.ms + e] * lc[r] : 0.0;
+                az[r] = fma(sv, zs[e], az[r]);
+                aw[r] = fma(sv, ws[e], aw[r]);
+                qf[r] = fma(sv, y[r], qf[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) {
+                az[r] += __shfl_xor(az[r], o);
+                aw[r] += __shfl_xor(aw[r], o);
+                qf[r] += __shfl_xor(qf[r], o);
+            }
+            if (col == r && row[r] < a.nobs) {
+                const double rs = a.sv[row[r]] * lc[r] - aw[r];
+                const int o = perm[row[r]];
+                const double sd = (double)estd[o];
+                const double d = sd * sqrt_rf[type[o]] * sqm;
+                atomicAdd(&gy[row[r]], az[r] * lc[r] / d);
+                atomicAdd(&gR[row[r]], (-az[r] * rs + qf[r]) / (sd * sd));
+            }
+        }
     }
 }
 
-__global__ void nonzero_rows_kernel(const double* __restrict__ g, int nrow, int width, int* __restrict__ flags,
-                                    int accumulate)
+__global__ void __launch_bounds__(256) nonzero_rows_kernel(const double* __restrict__ g, int nrow, int width,
+                                                           int* __restrict__ flags, int accumulate)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    // a wavefront per row, coalesced (a thread per row: 1.3 ms for 3,111 rows
+    // of 96 x 96)
+    const int r = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= nrow)
         return;
-    int nz = 0;
-    for (int e = 0; e < width; ++e)
-        nz |= g[(size_t)r * width + e] != 0.0;
-    flags[r] = accumulate ? (flags[r] | nz) : nz;
+    const double* row = g + (size_t)r * width;
+    bool nz = false;
+    for (int e0 = 0; e0 < width && !__any(nz); e0 += 512)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = e0 + 64 * u + lane;
+            nz |= e < width && row[e] != 0.0;
+        }
+    const int any = __any(nz) ? 1 : 0;
+    if (lane == 0)
+        flags[r] = accumulate ? (flags[r] | any) : any;
 }
 
 // sum over the 256 threads of a workgroup (fixed order: waves, then the
@@ -424,23 +471,40 @@ __global__ void __launch_bounds__(256) adj_B_kernel(CalcArgs a, const double* __
     const double* Dn = D + (size_t)node * md * m;
     double* Y = y + (size_t)k * MP * MP;
     double* Bk = B + (size_t)k * MP * MP;
-    for (int q = threadIdx.x; q < MP * MP; q += 256) {
-        const int r = q / MP, c = q - r * MP;
-        double s = 0.0;
-        if (r < md && c < m)
-            for (int b = 0; b < m; ++b)
-                s = fma(Dn[(size_t)r * m + b], mi[(size_t)b * MP + c], s);
-        Y[q] = s;
+    // tile products by FP64 MFMA, a wavefront taking output tiles w, w + 4, ...;
+    // k-step r of block K is members 16 K + 4 grp + r in both operands
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 15, grp = lane >> 4;
+    for (int t = wave; t < MT * MT; t += 4) {      // Y = D M^-1
+        const int I = t / MT, J = t % MT;
+        const int e1 = 16 * I + col;
+        tile4 y = {0.0, 0.0, 0.0, 0.0};
+        for (int K = 0; K < MT; ++K)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int b = 16 * K + 4 * grp + r;
+                const double d = (e1 < md && b < m) ? Dn[(size_t)e1 * m + b] : 0.0;
+                y = __builtin_amdgcn_mfma_f64_16x16x4f64(d, mi[(size_t)b * MP + 16 * J + col], y, 0, 0, 0);
+            }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            Y[(size_t)(16 * I + 4 * r + grp) * MP + 16 * J + col] = y[r];
     }
     __syncthreads();
     const double h = 0.5 * a.alpha;
-    for (int q = threadIdx.x; q < MP * MP; q += 256) {
-        const int r = q / MP, c = q - r * MP;
-        double s = 0.0;
-        if (r < m && c < m)
-            for (int e = 0; e < md; ++e)
-                s = fma(mi[(size_t)r * MP + e], Y[(size_t)e * MP + c], s);
-        Bk[q] = h * s;
+    for (int t = wave; t < MT * MT; t += 4) {      // B = alpha / 2 M^-1 Y (M^-1 symmetric)
+        const int I = t / MT, J = t % MT;
+        tile4 y = {0.0, 0.0, 0.0, 0.0};
+        for (int K = 0; K < MT; ++K)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int b = 16 * K + 4 * grp + r;
+                y = __builtin_amdgcn_mfma_f64_16x16x4f64(mi[(size_t)b * MP + 16 * I + col],
+                                                         Y[(size_t)b * MP + 16 * J + col], y, 0, 0, 0);
+            }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            Bk[(size_t)(16 * I + 4 * r + grp) * MP + 16 * J + col] = h * y[r];
     }
 }
 
@@ -450,7 +514,7 @@ hipError_t launch_nonzero_rows(hipStream_t s, const double* g, int nrow, int wid
 {
     if (nrow == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(nonzero_rows_kernel, dim3((unsigned)((nrow + 255) / 256)), dim3(256), 0, s, g, nrow, width,
+    hipLaunchKernelGGL(nonzero_rows_kernel, dim3((unsigned)((nrow + 3) / 4)), dim3(256), 0, s, g, nrow, width,
                        flags, accumulate ? 1 : 0);
     return hipGetLastError();
 }
@@ -502,19 +566,33 @@ hipError_t launch_adj_B(hipStream_t s, const CalcArgs& a, const double* D_nodes,
     return hipGetLastError();
 }
 
+// few nodes: their obs spread over more workgroups
+template <int MT>
+void launch_adj_obs_mt(hipStream_t s, const CalcArgs& a, const int* perm, const short* type, const float* estd,
+                       const double* sqrt_rfactor, const double* B, double* dJ_dy, double* dJ_dR)
+{
+    const int split = a.nbatch >= 1024 ? 1 : (a.nbatch >= 256 ? 4 : 16);
+    const dim3 grid((unsigned)a.nbatch, (unsigned)split);
+    if (B != nullptr)
+        hipLaunchKernelGGL((adj_obs_kernel<MT, true>), grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B,
+                           dJ_dy, dJ_dR);
+    else
+        hipLaunchKernelGGL((adj_obs_kernel<MT, false>), grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B,
+                           dJ_dy, dJ_dR);
+}
+
 hipError_t launch_adj_obs(hipStream_t s, const CalcArgs& a, const int* perm, const short* type, const float* estd,
                           const double* sqrt_rfactor, const double* B, double* dJ_dy, double* dJ_dR)
 {
     if (a.nbatch == 0)
         return hipSuccess;
-    const dim3 grid((unsigned)a.nbatch);
     switch ((a.m + 15) / 16) {
-    case 1: hipLaunchKernelGGL(adj_obs_kernel<1>, grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
-    case 2: hipLaunchKernelGGL(adj_obs_kernel<2>, grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
-    case 3: hipLaunchKernelGGL(adj_obs_kernel<3>, grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
-    case 4: hipLaunchKernelGGL(adj_obs_kernel<4>, grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
-    case 5: hipLaunchKernelGGL(adj_obs_kernel<5>, grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
-    case 6: hipLaunchKernelGGL(adj_obs_kernel<6>, grid, dim3(256), 0, s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
+    case 1: launch_adj_obs_mt<1>(s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
+    case 2: launch_adj_obs_mt<2>(s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
+    case 3: launch_adj_obs_mt<3>(s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
+    case 4: launch_adj_obs_mt<4>(s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
+    case 5: launch_adj_obs_mt<5>(s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
+    case 6: launch_adj_obs_mt<6>(s, a, perm, type, estd, sqrt_rfactor, B, dJ_dy, dJ_dR); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
