@@ -26,6 +26,14 @@ __host__ __device__ constexpr int item_groups_lo(int MT)
     return MT <= 4 ? 2 : (MT <= 6 ? 1 : (MT == 7 ? 3 : (MT <= 9 ? 4 : 5)));
 }
 
+// Launches of few nodes: about three tiles a wavefront, so that a list's
+// chunks take less time each and more wavefronts share the work (9 nodes of
+// four lists, the longest 3,000 obs, m = 96: 0.41 ms with two groups).  Used
+// where even then the items are fewer than kManyItems, two wavefronts per
+// SIMD; the matrices are the same bit for bit.
+__host__ __device__ constexpr int item_groups_many(int MT) { return MT <= 4 ? item_groups_lo(MT) + 1 : (tri_count(MT) + 2) / 3; }
+constexpr long long kManyItems = 2048;
+
 // The items (segment, tile group) of the item Gram kernels are dealt to the 8
 // XCDs in runs of kItemRun.  Block i runs on XCD i % 8 (the hardware
 // dispatcher deals blocks round-robin), and XCD x takes runs x, x + 8,

@@ -268,7 +268,9 @@ template <int M>
 void launch_mix_item(hipStream_t s, dim3 grid, const CalcArgs& a, int ng)
 {
     constexpr int lo = item_groups_lo(M);
-    if (ng == lo + 1)
+    if (ng == item_groups_many(M))
+        hipLaunchKernelGGL((gram_mixed_item_kernel<M, item_groups_many(M)>), grid, dim3(64), 0, s, a);
+    else if (ng == lo + 1)
         hipLaunchKernelGGL((gram_mixed_item_kernel<M, lo + 1>), grid, dim3(64), 0, s, a);
     else
         hipLaunchKernelGGL((gram_mixed_item_kernel<M, lo>), grid, dim3(64), 0, s, a);
@@ -283,7 +285,9 @@ hipError_t launch_gram_mixed(hipStream_t s, const CalcArgs& a)
         // tile groups per segment: one of the two candidates of this MT (the
         // smaller by default)
         const int lo = item_groups_lo(MT);
-        const int ng = (a.tile_groups == lo + 1) ? lo + 1 : lo;
+        const long long nlist = (long long)a.nbatch * a.nseg;
+        const int ng = nlist * item_groups_many(MT) <= kManyItems ? item_groups_many(MT)
+                                                                  : (a.tile_groups == lo + 1 ? lo + 1 : lo);
         const long long nitem = (long long)a.nbatch * a.nseg * ng;
         const dim3 igrid(item_grid(nitem));
         switch (MT) {
