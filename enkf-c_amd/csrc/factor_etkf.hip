@@ -23,7 +23,7 @@
 // the workspace's traffic (130 KB an inverse).  For m = 96 about 14 inverses
 // a node.  Measured against the kernel before it (pivots swept one per
 // workgroup barrier, one five-wave workgroup per CU): 51x1500x1800 tile FP64
-// calc 1,909 -> 756 ms; 4,050 nodes, m = 96: 21.0 -> 7.1 ms; 2,278 nodes, m =
+// calc 1,909 -> 561 ms; 4,050 nodes, m = 96: 21.0 -> 4.3 ms; 2,278 nodes, m =
 // 24: 0.61 -> 0.22 ms.  m > 96 had iterates in memory and Gauss-Jordan
 // inverses of up to 2 KB of spills a lane; it takes the same path now.
 #include <algorithm>
