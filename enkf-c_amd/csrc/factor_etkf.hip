@@ -9,8 +9,10 @@
 //   mu_k = |det Y_k det Z_k|^(-1/(2m))
 // whose two inverses are the block elimination of the DEnKF factorisation.
 // Y_k = M Z_k, so det Z_k = det Y_k / det M and mu_k is known from Y_k alone (in
-// single precision: any scaling near it converges as fast);
-// each inverse is combined tile by tile as it is formed.  The first step
+// single precision: any scaling near it converges as fast).  The padding (rows
+// m ..) is kept the identity in Y and Z, as it is in M: scaled with the rest, it
+// would enter the determinants, whose root is of order 2m, and for m <= 7 mu
+// runs away.  Each inverse is combined tile by tile as it is formed.  The first step
 // needs one inverse (Z_0 = I; it gives w, dfs and srf too), the last one
 // Y_k^-1 only.  Once a step changes Z by less than 1e-8 of its norm, one more
 // unscaled step is taken and is the last (the iteration converges
@@ -193,12 +195,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     eye[r] = (I == J && 4 * r + (l0 >> 4) == (l0 & 15)) ? 1.0 : 0.0;
+                // the last diagonal tile's columns m .. (elsewhere theirs stay 0)
+                const bool pad = I == J && I == MT - 1 && 16 * I + (l0 & 15) >= m;
                 if (z) {
                     o = eye;
                     // Y_1 = (mu M + I / mu) / 2
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        Y[at + 64 * r + l0] = hm * Y[at + 64 * r + l0] + hi * eye[r];
+                        Y[at + 64 * r + l0] = pad ? eye[r] : hm * Y[at + 64 * r + l0] + hi * eye[r];
                     mulb(ic, jc, v);
                     if (I == J) {
 #pragma unroll
@@ -214,11 +218,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    nv[r] = hm * o[r] + hi * v[r];
+                    nv[r] = pad ? eye[r] : hm * o[r] + hi * v[r];
                     const double d = nv[r] - o[r];
                     // off-diagonal tiles stand for themselves and their transposes
                     dn += (I == J ? 1.0 : 2.0) * d * d;
-                    nn += (I == J ? 1.0 : 2.0) * nv[r] * nv[r];
+                    nn += pad ? 0.0 : (I == J ? 1.0 : 2.0) * nv[r] * nv[r];
                 }
                 asm volatile("" : "+v"(dn), "+v"(nn), "+v"(trx));
                 if (tt) {

@@ -103,14 +103,12 @@ __device__ __attribute__((always_inline)) inline double rows_bcast(double v)
 // j > K.  Rows of x above and of f below K do not matter any more, or yet;
 // dcol receives the pivot in the lanes of column K.
 template <int K>
-__device__ __attribute__((always_inline)) inline void chol_pivot(tile4& x, tile4& f, double& dcol, int col, bool& bad,
-                                                                 double& det)
+__device__ __attribute__((always_inline)) inline void chol_pivot(tile4& x, tile4& f, double& dcol, int col, bool& bad)
 {
     constexpr int RK = K >> 2, GK = K & 3;
     const double p = rows_bcast<GK>(x[RK]);   // x_K,col
     const double d = row_bcast<K>(p);
     bad |= !(d > 0.0);
-    det *= d;
     dcol = col == K ? d : dcol;
     if constexpr (K < 15) {
         const double ws = col > K ? p * recip_pivot(d) : 0.0;
@@ -120,7 +118,7 @@ __device__ __attribute__((always_inline)) inline void chol_pivot(tile4& x, tile4
 #pragma unroll
         for (int r = 0; r <= RK; ++r)
             f[r] = fma(-row_bcast<K>(f[r]), ws, f[r]);
-        chol_pivot<K + 1>(x, f, dcol, col, bad, det);
+        chol_pivot<K + 1>(x, f, dcol, col, bad);
     }
 }
 
@@ -135,16 +133,16 @@ __device__ inline double rsqrt_pivot(double d)
 }
 
 // x <- W, upper triangular, W W^T = x^-1, for a symmetric positive definite
-// tile (x = R^T R, W = R^-1); det is its determinant
-__device__ __attribute__((always_inline)) inline void tile_chol(tile4& x, int lane, bool& bad, double& det)
+// tile (x = R^T R, W = R^-1); the lanes of column k add log2 of pivot k to ld
+__device__ __attribute__((always_inline)) inline void tile_chol(tile4& x, int lane, bool& bad, float& ld)
 {
     tile4 f;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         f[r] = (4 * r + (lane >> 4) == (lane & 15)) ? 1.0 : 0.0;
-    det = 1.0;
     double dcol = 1.0;
-    chol_pivot<0>(x, f, dcol, lane & 15, bad, det);
+    chol_pivot<0>(x, f, dcol, lane & 15, bad);
+    ld += __builtin_amdgcn_logf((float)__builtin_amdgcn_frexp_mant(dcol)) + (float)__builtin_amdgcn_frexp_exp(dcol);
     const double s = rsqrt_pivot(dcol);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -164,7 +162,9 @@ __host__ __device__ constexpr int tri_at(int i, int j)
 //
 //   R_kj = W_k^T A_kj;   A_ij += (-R_ki)^T R_kj,  k < i <= j
 //
-// log2det: log2 of the determinant, in single precision.
+// log2det: log2 of the determinant, in single precision: the sum of the
+// pivots' (their product leaves the range of a double where 16 of them exceed
+// 1e19).
 //
 // With the inverse of a triangular diagonal block the error stays within
 // cond(R_kk) of the unblocked elimination's; with the inverse of the block
@@ -173,16 +173,11 @@ __host__ __device__ constexpr int tri_at(int i, int j)
 template <int MT>
 __device__ __attribute__((always_inline)) inline void tile_eliminate(tile4* x, int lane, bool& bad, float& log2det)
 {
-    double mant = 1.0;
-    int ex = 0;
+    float ld = 0.0f;
     auto factor = [&](tile4& d) {
-        double det;
         int ln = lane;
         asm volatile("" : "+v"(ln));   // (the pivots' masks are not kept between them)
-        tile_chol(d, ln, bad, det);
-        int e;
-        mant = frexp(mant * det, &e);
-        ex += e;
+        tile_chol(d, ln, bad, ld);
     };
     auto eliminate = [&](auto kc, const tile4& d) {
         constexpr int k = kc;
@@ -233,7 +228,10 @@ __device__ __attribute__((always_inline)) inline void tile_eliminate(tile4* x, i
             });
         }
     }
-    log2det = __builtin_amdgcn_logf((float)mant) + (float)ex;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1)
+        ld += __shfl_xor(ld, o);
+    log2det = ld;
 }
 
 // After tile_eliminate: tile (i, j), i <= j, becomes V_ji of the lower

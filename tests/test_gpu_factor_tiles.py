@@ -51,3 +51,37 @@ def test_factor_tiles_mixed(m):
     move by that times the condition of M, below 100 here."""
     print("case factor tiles mixed m=%d" % m, flush=True)
     check(m, enkfg.PREC_MIXED, 2e-3, 2e-3, 2e-3)
+
+
+@pytest.mark.parametrize("errscale", [1.0, 1e-2, 1e-4])
+@pytest.mark.parametrize("m", [2, 3, 5, 7, 8, 15, 16, 17, 33, 48, 64, 65, 80, 81, 97, 112, 113, 128, 129, 145])
+def test_factor_etkf_sizes(m, errscale):
+    """ETKF (factor_etkf.hip): T = M^-1/2 and w = M^-1 S^T s against the
+    eigen-decomposition of M from the oracle's lists, for member counts that
+    fill their tiles or leave most of the last one empty, and observation
+    errors down to 1e-4 of the ensemble's spread.  The rounding of the sums in
+    M, m eps |M|, moves T by that times |M^-1| <= 1 and w by that times |w|,
+    and that of S^T s moves w; four times that is allowed."""
+    print("case etkf m=%d errscale=%g" % (m, errscale), flush=True)
+    P = synth.make_problem(seed=m, nmem=m, nobs=700, nj=16, ni=20, nk=3, locrad=60.0, stride=4, profiles=40)
+    estd = (P.obs_estd * errscale).astype(np.float32)
+    ob = O.OracleObs(P.obstypes, P.obs_type, P.obs_lon, P.obs_lat, estd)
+    S, s = O.standardise(m, ob, P.HA, P.innov)
+    E = enkfg.Engine(m, scheme=enkfg.SCHEME_ETKF, keep_fp64=True)
+    E.set_obstypes(P.obstypes)
+    E.set_obs(P.obs_type, P.obs_status, P.obs_lon, P.obs_lat, estd)
+    E.set_S(P.HA, P.innov, standardised=False)
+    E.calc_transforms(P.node_lon, P.node_lat, stride=P.stride)
+    T, w, T64, w64 = E.transforms(fp64=True)
+    E.close()
+    T64, w64 = T64.reshape(-1, m, m), w64.reshape(-1, m)
+    eps = np.finfo(np.float64).eps
+    for k, (lo, la) in enumerate(zip(P.node_lon.ravel(), P.node_lat.ravel())):
+        ids, lc = ob.findlocal(lo, la)
+        A = S[:, ids].astype(np.float64) * lc
+        b = A @ (s[ids] * lc)
+        lam, V = np.linalg.eigh(np.eye(m) + A @ A.T)
+        tol = 4 * m * eps * lam[-1]
+        assert np.abs(T64[k] - (V / np.sqrt(lam)) @ V.T).max() <= tol
+        wr = (V / lam) @ (V.T @ b)
+        assert np.abs(w64[k] - wr).max() <= tol * np.abs(wr).max() + 4 * m * eps * (np.abs(A) @ np.abs(s[ids] * lc)).max()
