@@ -129,6 +129,7 @@ struct enkfg_ctx {
     DevBuf d_raw, d_rawoff, d_rrow, d_rd2, d_srow, d_sd2;   // NLOBSMAX candidates
     DevBuf d_lflag;               // box search: an obs lies at exactly a radius
     bool lists_valid = false;
+    int list_ni = 0, list_nj = 0; // the node grid they belong to (enkfg_set_transforms brings another ni_s, nj_s)
     bool lists_ordered = false;   // the lists are in the reference's order
     bool lists_vis = false;       // they were made with the visibility mask in d_vis
 
@@ -480,7 +481,7 @@ int ensure_trees(enkfg_ctx* c)
 // the lists filled in the reference's order, their offsets known
 hipError_t fill_ordered(enkfg_ctx* c, bool nlobsmax)
 {
-    return launch_loc_fill(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
+    return launch_loc_fill(c->stream, c->list_ni, c->list_nj, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
                            c->lists_vis ? c->d_vis.as<unsigned char>() : nullptr, c->d_nodes.as<KdNode>(),
                            c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), (int)c->types.size(),
                            c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_offsets.as<long long>(),
@@ -506,6 +507,8 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
     int r = node_inputs(c, nodes);
     if (r != ENKFG_OK)
         return r;
+    c->list_ni = nodes->ni;
+    c->list_nj = nodes->nj;
     const int nt = (int)c->types.size();
     const long long ncnt = (long long)c->nnode * nt;
     HIPCHECK(c, c->d_counts.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
@@ -1195,6 +1198,9 @@ int enkfg_get_local_counts(enkfg_ctx* c, int* counts)
         return ENKFG_ERR_ARG;
     if (!c->lists_valid || counts == nullptr)
         return fail(c, ENKFG_ERR_STATE, "no local lists");
+    if (c->nnode > (long long)c->list_ni * c->list_nj)
+        return fail(c, ENKFG_ERR_STATE, "the local lists are of %d x %d nodes, fewer than the transforms'", c->list_nj,
+                    c->list_ni);
     const int nt = (int)c->types.size();
     std::vector<long long> off(c->nnode + 1);
     for (int k = 0; k <= c->nnode; ++k)
@@ -1211,7 +1217,7 @@ int enkfg_get_localobs(enkfg_ctx* c, int node, int cap, int* ids, double* lc)
         return ENKFG_ERR_ARG;
     if (!c->lists_valid)
         return fail(c, ENKFG_ERR_STATE, "no local lists");
-    if (node < 0 || node >= c->nnode)
+    if (node < 0 || node >= c->nnode || node >= (long long)c->list_ni * c->list_nj)
         return fail(c, ENKFG_ERR_ARG, "node out of range");
     const int nt = (int)c->types.size();
     long long o[2];
@@ -2287,6 +2293,8 @@ int enkfg_adjoint(enkfg_ctx* c, const float* dev_dJ_dmean, double* dJ_dy, double
         return fail(c, ENKFG_ERR_ARG, "dJ/dmean is NULL");
     if (!c->S_set || !c->lists_valid || !c->transforms_valid)
         return fail(c, ENKFG_ERR_STATE, "the adjoint needs S, and enkfg_calc_transforms on the same grid");
+    if (c->list_ni != c->ni_s || c->list_nj != c->nj_s)
+        return fail(c, ENKFG_ERR_STATE, "the local lists are of another node grid than the transforms");
     if (c->attached_E == nullptr)
         return fail(c, ENKFG_ERR_STATE, "the adjoint needs the forecast ensemble attached (enkfg_ens_attach)");
     const int m = c->cfg.nmem;
@@ -2398,6 +2406,8 @@ int enkfg_adjoint_ens(enkfg_ctx* c, const float* dev_dJ_dXa, double* dJ_dy, doub
         return fail(c, ENKFG_ERR_ARG, "dJ/dXa is NULL");
     if (!c->S_set || !c->lists_valid || !c->transforms_valid)
         return fail(c, ENKFG_ERR_STATE, "the adjoint needs S, and enkfg_calc_transforms on the same grid");
+    if (c->list_ni != c->ni_s || c->list_nj != c->nj_s)
+        return fail(c, ENKFG_ERR_STATE, "the local lists are of another node grid than the transforms");
     if (c->attached_E == nullptr)
         return fail(c, ENKFG_ERR_STATE, "the adjoint needs the forecast ensemble attached (enkfg_ens_attach)");
     if (c->cfg.mode == ENKFG_MODE_ENOI)

@@ -1,0 +1,56 @@
+"""The local lists between calls, through the C ABI: which node grid they
+belong to, what reads them, and what leaves them as they are."""
+import numpy as np
+import pytest
+
+import enkfg
+import oracle as O
+import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def setup(nmem=8, **kw):
+    P = synth.make_problem(**dict(dict(seed=3, nmem=nmem, nobs=1500, nj=24, ni=30, nk=2, locrad=80.0, stride=3), **kw))
+    E = enkfg.Engine(nmem, keep_fp64=True)
+    E.set_obstypes(P.obstypes)
+    E.set_obs(P.obs_type, P.obs_status, P.obs_lon, P.obs_lat, P.obs_estd)
+    E.set_S(P.HA, P.innov, standardised=False)
+    ob = O.OracleObs(P.obstypes, P.obs_type, P.obs_lon, P.obs_lat, P.obs_estd)
+    return P, E, ob
+
+
+def check_lists(E, ob, lon, lat, nodes):
+    for k in nodes:
+        ids, lc = ob.findlocal(lon.ravel()[k], lat.ravel()[k])
+        got = E.localobs(k, len(ids))
+        assert np.array_equal(got[0][:len(ids)], ids) and np.array_equal(got[1][:len(ids)], lc)
+
+
+@pytest.mark.parametrize("ordered", [False, True])
+def test_lists_keep_their_grid_when_transforms_are_set(ordered):
+    """enkfg_set_transforms brings a node grid of its own; the lists of the
+    calc (or of enkfg_localise) before it stay those of their nodes."""
+    print("case lists and set_transforms ordered=%d" % ordered, flush=True)
+    P, E, ob = setup()
+    if ordered:
+        E.calc_transforms(P.node_lon, P.node_lat, stride=P.stride)
+        E.localise(P.node_lon, P.node_lat, stride=P.stride)
+    else:
+        E.calc_transforms(P.node_lon, P.node_lat, stride=P.stride)
+    nn = P.node_lon.size
+    counts = E.local_counts()
+    m = E.nmem
+    for nj, ni in ((40, 50), (2, 3)):
+        E.set_transforms(np.zeros((nj, ni, m, m), np.float32), np.zeros((nj, ni, m), np.float32), P.stride)
+        check_lists(E, ob, P.node_lon, P.node_lat, range(min(nn, nj * ni)))
+        for bad in (nn, nj * ni) if nn > nj * ni else (nn, nj * ni - 1, nj * ni):
+            with pytest.raises(enkfg.EnkfgError):
+                E.localobs(bad, 10000)
+    E.nnode = 2 * 3
+    assert np.array_equal(E.local_counts(), counts[:6])
+    E.set_transforms(np.zeros((40, 50, m, m), np.float32), np.zeros((40, 50, m), np.float32), P.stride)
+    E.nnode = 40 * 50
+    with pytest.raises(enkfg.EnkfgError):
+        E.local_counts()
+    E.close()
