@@ -91,6 +91,11 @@ void ll2xyz(double lon_deg, double lat_deg, double* out)
 constexpr int kBuckets = 4;
 constexpr int kBucketLo[kBuckets] = {0, 256, 1024, 4096};
 
+// nodes whose lists are ordered together for enkfg_get_localobs, at first,
+// and list entries of a run beyond that (3 GB)
+constexpr int kOrderRun = 1024;
+constexpr long long kOrderEntries = 1LL << 28;
+
 struct enkfg_ctx {
     enkfg_config cfg{};
     std::string err;
@@ -132,6 +137,12 @@ struct enkfg_ctx {
     int list_ni = 0, list_nj = 0; // the node grid they belong to (enkfg_set_transforms brings another ni_s, nj_s)
     bool lists_ordered = false;   // the lists are in the reference's order
     bool lists_vis = false;       // they were made with the visibility mask in d_vis
+    // otherwise: the lists of run_n nodes from run_node0 in that order, for
+    // enkfg_get_localobs; entry run_off0 of all lists is their first
+    DevBuf d_run_ids, d_run_lc;
+    int run_node0 = 0, run_n = 0;
+    int run_next = 0;             // nodes of the next run
+    long long run_off0 = 0;
 
     // calc batching: nodes ordered by obs-count bucket (heaviest first), and
     // the autotuned Gram tile groups per [precision][bucket] (0 = not tuned)
@@ -490,6 +501,47 @@ hipError_t fill_ordered(enkfg_ctx* c, bool nlobsmax)
                            nlobsmax ? c->d_sd2.as<double>() : nullptr);
 }
 
+// The lists of `node` and of its neighbours in the reference's order, in a
+// buffer of their own: the calc's lists stay as they are.  A walk is a
+// thread's serial chain and takes about as long for a thousand nodes as for
+// one (12 ms for 9 nodes of 200 x 240 cells; 540x801 cells: 17 ms for 1,024
+// nodes, 31 for all 48,060), so the first run takes kOrderRun nodes and each
+// further one eight times as many, for callers that read the whole grid.
+int order_run(enkfg_ctx* c, int node)
+{
+    int r = ensure_trees(c);
+    if (r != ENKFG_OK)
+        return r;
+    const int nt = (int)c->types.size();
+    const int nn = c->list_ni * c->list_nj;
+    int node0, n;
+    long long o[2];
+    for (;; c->run_next /= 8) {
+        node0 = node / c->run_next * c->run_next;
+        n = std::min(c->run_next, nn - node0);
+        for (int k = 0; k < 2; ++k)
+            HIPCHECK(c, hipMemcpy(&o[k], c->d_offsets.as<long long>() + (size_t)(node0 + k * n) * nt, sizeof(long long),
+                                  hipMemcpyDeviceToHost));
+        if (o[1] - o[0] <= kOrderEntries || c->run_next <= kOrderRun)
+            break;
+    }
+    c->run_n = 0;
+    const long long off0 = o[0] / 8 * 8;   // (whole bursts stay aligned)
+    HIPCHECK(c, c->d_run_ids.reserve((size_t)(o[1] - off0) * sizeof(int)));
+    HIPCHECK(c, c->d_run_lc.reserve((size_t)(o[1] - off0) * sizeof(double)));
+    HIPCHECK(c, launch_loc_fill_run(c->stream, node0, n, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
+                                    c->lists_vis ? c->d_vis.as<unsigned char>() : nullptr, c->d_nodes.as<KdNode>(),
+                                    c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(),
+                                    c->d_obsids.as<int>(), c->d_offsets.as<long long>(), off0, c->d_run_ids.as<int>(),
+                                    c->d_run_lc.as<double>()));
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    c->run_node0 = node0;
+    c->run_n = n;
+    c->run_next = (int)std::min<long long>(8LL * c->run_next, 1 << 30);
+    c->run_off0 = off0;
+    return ENKFG_OK;
+}
+
 // The lists of every node.  The box search counts them; it fills them too
 // unless the caller wants the reference's order (ordered), for which the
 // trees are walked.  The trees decide alone where the box search does not
@@ -504,6 +556,8 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
         if (t.nlobsmax != ENKFG_NLOBSMAX_NONE)
             nlobsmax = true;
     c->lists_valid = false;
+    c->run_n = 0;
+    c->run_next = kOrderRun;
     int r = node_inputs(c, nodes);
     if (r != ENKFG_OK)
         return r;
@@ -682,7 +736,7 @@ void enkfg_destroy(enkfg_ctx* c)
         (void)hipStreamSynchronize(c->stream2);
     DevBuf* bufs[] = {&c->d_nodes, &c->d_types, &c->d_obsids, &c->d_type, &c->d_status, &c->d_estd, &c->d_sqrtrf,
                       &c->d_perm, &c->d_S, &c->d_s, &c->d_tmp, &c->d_tmp2, &c->d_qxyz, &c->d_glob, &c->d_vis, &c->d_counts, &c->d_offsets,
-                      &c->d_scantmp, &c->d_ids, &c->d_lc, &c->d_lflag, &c->d_noderow, &c->d_xyz, &c->d_boxes,
+                      &c->d_scantmp, &c->d_ids, &c->d_lc, &c->d_run_ids, &c->d_run_lc, &c->d_lflag, &c->d_noderow, &c->d_xyz, &c->d_boxes,
                       &c->d_raw, &c->d_rawoff, &c->d_rrow, &c->d_rd2,
                       &c->d_srow, &c->d_sd2, &c->d_T, &c->d_w, &c->d_T64, &c->d_w64, &c->d_pnlobs,
                       &c->d_pdfs, &c->d_psrf, &c->d_gram, &c->d_order, &c->d_segord, &c->d_sts, &c->d_err, &c->d_E, &c->d_infl, &c->d_nlev,
@@ -1228,23 +1282,26 @@ int enkfg_get_localobs(enkfg_ctx* c, int node, int cap, int* ids, double* lc)
     const long long p = o[1] - o[0];
     if (p > cap)
         return fail(c, ENKFG_ERR_ARG, "cap %d < %lld local obs", cap, p);
-    if (p > 0 && !c->lists_ordered) {
-        // the calc's lists are in row order; the caller's in the reference's
-        int r = ensure_trees(c);
-        if (r != ENKFG_OK)
-            return r;
-        HIPCHECK(c, fill_ordered(c, false));
-        HIPCHECK(c, hipStreamSynchronize(c->stream));
-        c->lists_ordered = true;
-    }
     if (p > 0) {
+        const int* dids = c->d_ids.as<int>() + o[0];
+        const double* dlc = c->d_lc.as<double>() + o[0];
+        if (!c->lists_ordered) {
+            // the calc's lists are in row order; the caller's in the reference's
+            if (node < c->run_node0 || node - c->run_node0 >= c->run_n) {
+                const int r = order_run(c, node);
+                if (r != ENKFG_OK)
+                    return r;
+            }
+            dids = c->d_run_ids.as<int>() + (o[0] - c->run_off0);
+            dlc = c->d_run_lc.as<double>() + (o[0] - c->run_off0);
+        }
         if (ids != nullptr) {
-            HIPCHECK(c, hipMemcpy(ids, c->d_ids.as<int>() + o[0], p * sizeof(int), hipMemcpyDeviceToHost));
+            HIPCHECK(c, hipMemcpy(ids, dids, p * sizeof(int), hipMemcpyDeviceToHost));
             for (long long k = 0; k < p; ++k)
                 ids[k] = c->perm[ids[k]];   // device row -> obs index
         }
         if (lc != nullptr)
-            HIPCHECK(c, hipMemcpy(lc, c->d_lc.as<double>() + o[0], p * sizeof(double), hipMemcpyDeviceToHost));
+            HIPCHECK(c, hipMemcpy(lc, dlc, p * sizeof(double), hipMemcpyDeviceToHost));
     }
     return (int)ENKFG_OK;
 }

@@ -70,6 +70,12 @@ hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, co
                            const unsigned char* visible, const KdNode* nodes, const int* noderow,
                            const TypeInfo* types, int ntypes, const short* status, const int* obsids, const long long* offsets, int* ids,
                            double* lc, const long long* rawoff, const int* raw, const int* srow, const double* sd2);
+// the lists of nodes node0 .. node0 + n - 1 alone (no NLOBSMAX type), entry
+// off0 (a multiple of 8) of all lists at ids[0], lc[0]
+hipError_t launch_loc_fill_run(hipStream_t s, int node0, int n, const double* qxyz, const unsigned char* isglobal,
+                               const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                               const TypeInfo* types, int ntypes, const short* status, const int* obsids,
+                               const long long* offsets, long long off0, int* ids, double* lc);
 hipError_t launch_scan_counts(hipStream_t s, const int* counts, long long* offsets, long long n, void* tmp,
                               size_t* tmp_bytes);
 

@@ -399,7 +399,8 @@ __global__ void __launch_bounds__(256) loc_sort_big_kernel(int nnode, const Type
 // stores from 64 threads walking different lists leave their cache lines
 // part-written, and such lines are written back to memory several times over
 // (174 against 105 ms per localisation of the 51x1500x1800 tile; runs of 4
-// gave 118 ms, of 16 106 ms).
+// gave 118 ms, of 16 106 ms).  Nodes node0 .. nodeend - 1; ids and lc start at
+// list entry off0 (a multiple of kLocBurst).
 constexpr int kLocBurst = 8;
 
 __global__ void __launch_bounds__(64) loc_fill_kernel(int nnode, int ni, const double* __restrict__ qxyz,
@@ -413,17 +414,20 @@ __global__ void __launch_bounds__(64) loc_fill_kernel(int nnode, int ni, const d
                                                        const long long* __restrict__ offsets, int* __restrict__ ids,
                                                        double* __restrict__ lc, const long long* __restrict__ rawoff,
                                                        const int* __restrict__ raw, const int* __restrict__ srow,
-                                                       const double* __restrict__ sd2)
+                                                       const double* __restrict__ sd2, int node0, int nodeend, long long off0)
 {
     int t, node;
     if (!thread_node(nnode, ni, ntypes, t, node))
+        return;
+    node += node0;
+    if (node >= nodeend)
         return;
     double q[3] = {qxyz[3 * (size_t)node], qxyz[3 * (size_t)node + 1], qxyz[3 * (size_t)node + 2]};
     const bool glob = isglobal[node] != 0;
     const TypeInfo& ti = types[t];
     if (!ti.searchable || !(visible == nullptr || visible[t]))
         return;
-    long long o = offsets[(size_t)node * ntypes + t];
+    long long o = offsets[(size_t)node * ntypes + t] - off0;
     if (glob) {
         for (int i = 0; i < ti.nids; ++i) {
             ids[o + i] = obsids[ti.obsid0 + i];
@@ -833,7 +837,25 @@ hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, co
     if (nt <= 0)
         return hipSuccess;
     hipLaunchKernelGGL(loc_fill_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
-                       visible, nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, rawoff, raw, srow, sd2);
+                       visible, nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, rawoff, raw, srow, sd2,
+                       0, ni * nj, 0LL);
+    return hipGetLastError();
+}
+
+hipError_t launch_loc_fill_run(hipStream_t s, int node0, int n, const double* qxyz, const unsigned char* isglobal,
+                               const unsigned char* visible, const KdNode* nodes, const int* noderow,
+                               const TypeInfo* types, int ntypes, const short* status, const int* obsids,
+                               const long long* offsets, long long off0, int* ids, double* lc)
+{
+    if (n <= 0 || ntypes <= 0)
+        return hipSuccess;
+    if (off0 % kLocBurst != 0)
+        return hipErrorInvalidValue;
+    // rows of eight nodes: a tile of thread_node is 64 nodes of the run
+    const int nj = (n + 7) / 8;
+    hipLaunchKernelGGL(loc_fill_kernel, walk_grid(8, nj, ntypes), dim3(64), 0, s, 8 * nj, 8, qxyz, isglobal, visible,
+                       nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, nullptr, nullptr, nullptr,
+                       nullptr, node0, node0 + n, off0);
     return hipGetLastError();
 }
 

@@ -2,6 +2,7 @@
 belong to, what reads them, and what leaves them as they are."""
 import numpy as np
 import pytest
+import torch
 
 import enkfg
 import oracle as O
@@ -53,4 +54,36 @@ def test_lists_keep_their_grid_when_transforms_are_set(ordered):
     E.nnode = 40 * 50
     with pytest.raises(enkfg.EnkfgError):
         E.local_counts()
+    E.close()
+
+
+def test_reading_a_list_leaves_the_calc_lists():
+    """enkfg_get_localobs after a calc gives the list in the reference's order
+    and leaves the lists that the adjoint sums over as they are: one column,
+    one node, so that no sum depends on the order of atomics."""
+    print("case lists read between two adjoints", flush=True)
+    P, E, ob = setup(locrad=400.0)
+    lon, lat = P.node_lon[4:5, 5:6].copy(), P.node_lat[4:5, 5:6].copy()
+    E.calc_transforms(lon, lat)
+    X = torch.randn(1, 1, E.nmem, device="cuda") + 10.0
+    dJ = torch.ones(1, 1, device="cuda")
+    E.ens_attach(np.ones((1, 1), np.int32), 1, 0, 0, [dict(level=0)], X.data_ptr())
+    before = E.adjoint(dJ.data_ptr(), P.nobs)
+    assert E.local_counts()[0] > 1000 and np.abs(before[0]).max() > 0
+    check_lists(E, ob, lon, lat, [0])
+    after = E.adjoint(dJ.data_ptr(), P.nobs)
+    assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
+    E.close()
+
+
+def test_lists_read_across_runs():
+    """1,961 nodes (more than the 1,024 that are ordered together at first, no
+    multiple of 8), some without coordinates, read in no order."""
+    print("case lists read across runs", flush=True)
+    P, E, ob = setup(nj=111, ni=157)
+    lon, lat = P.node_lon.copy(), P.node_lat
+    assert lon.shape == (37, 53)
+    lon[0, 7] = lon[30, 5] = lon[36, 52] = np.nan
+    E.calc_transforms(lon, lat, stride=P.stride)
+    check_lists(E, ob, lon, lat, [1960, 0, 7, 1023, 1024, 1025, 1599, 63, 64, 1959, 1952, 1951, 1023, 1595, 1960])
     E.close()
