@@ -111,7 +111,7 @@ struct enkfg_ctx {
     std::vector<short> otype, ostatus;
     std::vector<float> olon, olat, oestd;
     bool obs_set = false;
-    DevBuf d_nodes, d_noderow, d_types, d_obsids, d_type, d_status, d_estd, d_sqrtrf, d_perm, d_xyz, d_boxes;
+    DevBuf d_nodes, d_noderow, d_rownode, d_types, d_obsids, d_type, d_status, d_estd, d_sqrtrf, d_perm, d_xyz, d_boxes;
     std::vector<TypeInfo> tinfo;
     // Device rows of S, s and status are ordered along a Morton curve (type by
     // type), so the obs near a node are a few runs of nearby rows; perm[row]
@@ -119,8 +119,7 @@ struct enkfg_ctx {
     // obs indices.
     std::vector<int> perm;
     size_t nsearch = 0;           // rows that are searched (the types' rows come first)
-    bool box_ok = false;          // finite coordinates only: the box search applies
-    bool trees_built = false;     // d_nodes, d_noderow hold the reference's trees
+    bool trees_built = false;     // d_nodes, d_noderow, d_rownode hold the reference's trees
 
     // S and s
     DevBuf d_S, d_s, d_tmp, d_tmp2;
@@ -132,7 +131,7 @@ struct enkfg_ctx {
     int node_geo = 0;
     DevBuf d_qxyz, d_glob, d_vis, d_counts, d_offsets, d_scantmp, d_ids, d_lc;
     DevBuf d_raw, d_rawoff, d_rrow, d_rd2, d_srow, d_sd2;   // NLOBSMAX candidates
-    DevBuf d_lflag;               // box search: an obs lies at exactly a radius
+    DevBuf d_lflag;               // box search: an obs lies a whole radius away along an axis
     bool lists_valid = false;
     int list_ni = 0, list_nj = 0; // the node grid they belong to (enkfg_set_transforms brings another ni_s, nj_s)
     bool lists_ordered = false;   // the lists are in the reference's order
@@ -235,7 +234,7 @@ unsigned long long spread3(unsigned long long v)
 
 // order[k]: the k-th of the n points (xyz[3 i ..]) along a Morton curve over
 // their bounding cube, equal codes in index order (a stable radix sort).
-// Points with a non-finite coordinate sort as if it were the lowest.
+// A coordinate that is not a number, or below all, sorts as the lowest.
 void morton_order(const std::vector<double>& xyz, int n, std::vector<int>& order)
 {
     double lo[3], ext = 0.0;
@@ -454,7 +453,7 @@ int ensure_trees(enkfg_ctx* c)
     for (int r = 0; r < c->nobs; ++r)
         rowof[(size_t)c->perm[(size_t)r]] = r;
     std::vector<KdNode> dnodes(c->nsearch);
-    std::vector<int> noderow(c->nsearch);
+    std::vector<int> noderow(c->nsearch), rownode(c->nsearch);   // (a type's nodes are counted from its first)
     for (size_t t = 0; t < c->tinfo.size(); ++t) {
         const TypeInfo& ti = c->tinfo[t];
         std::vector<int> ids(c->perm.begin() + ti.node0, c->perm.begin() + ti.node0 + ti.nnode);
@@ -476,14 +475,18 @@ int ensure_trees(enkfg_ctx* c)
             d.z = b.z;
             d.right = b.right;
             d.link = (unsigned)(b.parent + 1) | (b.left >= 0 ? 0x80000000u : 0u);
-            noderow[(size_t)ti.node0 + v] = rowof[(size_t)b.obsid];
+            const int row = rowof[(size_t)b.obsid];
+            noderow[(size_t)ti.node0 + v] = row;
+            rownode[(size_t)row] = v;
         }
     }
     HIPCHECK(c, c->d_nodes.reserve(std::max<size_t>(dnodes.size(), 1) * sizeof(KdNode)));
     HIPCHECK(c, c->d_noderow.reserve(std::max<size_t>(noderow.size(), 1) * sizeof(int)));
+    HIPCHECK(c, c->d_rownode.reserve(std::max<size_t>(rownode.size(), 1) * sizeof(int)));
     if (!dnodes.empty()) {
         HIPCHECK(c, hipMemcpy(c->d_nodes.p, dnodes.data(), dnodes.size() * sizeof(KdNode), hipMemcpyHostToDevice));
         HIPCHECK(c, hipMemcpy(c->d_noderow.p, noderow.data(), noderow.size() * sizeof(int), hipMemcpyHostToDevice));
+        HIPCHECK(c, hipMemcpy(c->d_rownode.p, rownode.data(), rownode.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     c->trees_built = true;
     return ENKFG_OK;
@@ -544,9 +547,7 @@ int order_run(enkfg_ctx* c, int node)
 
 // The lists of every node.  The box search counts them; it fills them too
 // unless the caller wants the reference's order (ordered), for which the
-// trees are walked.  The trees decide alone where the box search does not
-// apply: NLOBSMAX types, non-finite coordinates, and an observation at
-// exactly the radius (which counting finds).
+// trees are walked.  NLOBSMAX types are the trees' alone.
 int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
 {
     if (!c->obs_set)
@@ -574,57 +575,66 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
     HIPCHECK(c, launch_scan_counts(c->stream, nullptr, nullptr, ncnt, nullptr, &tmpb));
     HIPCHECK(c, c->d_scantmp.reserve(tmpb));
     tmpb = c->d_scantmp.bytes;
+    if (nlobsmax || ordered) {
+        r = ensure_trees(c);
+        if (r != ENKFG_OK)
+            return r;
+    }
     HIPCHECK(c, hipEventRecord(c->ev[0], c->stream));
-    bool boxes = c->box_ok && !nlobsmax;
     long long total = 0;
-    if (boxes) {
-        int tie = 0;
+    const auto box = [&](bool fill) {
+        const bool trees = c->trees_built;
+        return launch_loc_box(c->stream, c->list_ni, c->list_nj, c->d_qxyz.as<double>(),
+                              c->d_glob.as<unsigned char>(), vis, c->d_types.as<TypeInfo>(), nt,
+                              c->d_boxes.as<LocBox>(), c->d_xyz.as<double>(), c->nsearch, c->d_status.as<short>(),
+                              c->d_obsids.as<int>(), trees ? c->d_nodes.as<KdNode>() : nullptr,
+                              trees ? c->d_rownode.as<int>() : nullptr, c->d_counts.as<int>(), c->d_lflag.as<int>(),
+                              c->d_offsets.as<long long>(), fill ? c->d_ids.as<int>() : nullptr,
+                              fill ? c->d_lc.as<double>() : nullptr);
+    };
+    for (int tie = nlobsmax ? 0 : 1; tie != 0;) {   // again with the trees if there are ties
+        const bool trees = c->trees_built;
         HIPCHECK(c, hipMemsetAsync(c->d_lflag.p, 0, sizeof(int), c->stream));
-        HIPCHECK(c, launch_loc_box(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
-                                   vis, c->d_types.as<TypeInfo>(), nt, c->d_boxes.as<LocBox>(), c->d_xyz.as<double>(),
-                                   c->nsearch, c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_counts.as<int>(),
-                                   c->d_lflag.as<int>(), nullptr, nullptr, nullptr));
+        HIPCHECK(c, box(false));
         HIPCHECK(c, launch_scan_counts(c->stream, c->d_counts.as<int>(), c->d_offsets.as<long long>(), ncnt,
                                        c->d_scantmp.p, &tmpb));
         HIPCHECK(c, hipMemcpyAsync(&total, c->d_offsets.as<long long>() + ncnt, sizeof total, hipMemcpyDeviceToHost,
                                    c->stream));
         HIPCHECK(c, hipMemcpyAsync(&tie, c->d_lflag.p, sizeof tie, hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
-        boxes = tie == 0;
+        if (trees)
+            break;
+        if (tie != 0) {
+            r = ensure_trees(c);
+            if (r != ENKFG_OK)
+                return r;
+        }
     }
-    if (!boxes || ordered) {
-        r = ensure_trees(c);
-        if (r != ENKFG_OK)
-            return r;
-    }
-    if (!boxes) {
-        if (nlobsmax)
-            HIPCHECK(c, c->d_raw.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
+    if (nlobsmax) {
+        HIPCHECK(c, c->d_raw.reserve(std::max<long long>(ncnt, 1) * sizeof(int)));
         HIPCHECK(c, launch_loc_count(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(),
                                      c->d_glob.as<unsigned char>(), vis, c->d_nodes.as<KdNode>(),
                                      c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(),
-                                     c->d_counts.as<int>(), nlobsmax ? c->d_raw.as<int>() : nullptr));
-        if (nlobsmax) {
-            // NLOBSMAX types: candidates in visiting order, sorted by distance,
-            // the first NLOBSMAX with status OK kept (observations.c:1899-1908)
-            HIPCHECK(c, c->d_rawoff.reserve((ncnt + 1) * sizeof(long long)));
-            HIPCHECK(c, launch_scan_counts(c->stream, c->d_raw.as<int>(), c->d_rawoff.as<long long>(), ncnt,
-                                           c->d_scantmp.p, &tmpb));
-            long long nraw = 0;
-            HIPCHECK(c, hipMemcpyAsync(&nraw, c->d_rawoff.as<long long>() + ncnt, sizeof nraw, hipMemcpyDeviceToHost,
-                                       c->stream));
-            HIPCHECK(c, hipStreamSynchronize(c->stream));
-            HIPCHECK(c, c->d_rrow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
-            HIPCHECK(c, c->d_srow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
-            HIPCHECK(c, c->d_rd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
-            HIPCHECK(c, c->d_sd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
-            HIPCHECK(c, launch_loc_nlobsmax(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(),
-                                            c->d_glob.as<unsigned char>(), vis, c->d_nodes.as<KdNode>(),
-                                            c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt,
-                                            c->d_status.as<short>(), c->d_raw.as<int>(), c->d_rawoff.as<long long>(),
-                                            c->d_rrow.as<int>(), c->d_rd2.as<double>(), c->d_srow.as<int>(),
-                                            c->d_sd2.as<double>(), c->d_counts.as<int>()));
-        }
+                                     c->d_counts.as<int>(), c->d_raw.as<int>()));
+        // NLOBSMAX types: candidates in visiting order, sorted by distance,
+        // the first NLOBSMAX with status OK kept (observations.c:1899-1908)
+        HIPCHECK(c, c->d_rawoff.reserve((ncnt + 1) * sizeof(long long)));
+        HIPCHECK(c, launch_scan_counts(c->stream, c->d_raw.as<int>(), c->d_rawoff.as<long long>(), ncnt,
+                                       c->d_scantmp.p, &tmpb));
+        long long nraw = 0;
+        HIPCHECK(c, hipMemcpyAsync(&nraw, c->d_rawoff.as<long long>() + ncnt, sizeof nraw, hipMemcpyDeviceToHost,
+                                   c->stream));
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        HIPCHECK(c, c->d_rrow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
+        HIPCHECK(c, c->d_srow.reserve(std::max<long long>(nraw, 1) * sizeof(int)));
+        HIPCHECK(c, c->d_rd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
+        HIPCHECK(c, c->d_sd2.reserve(std::max<long long>(nraw, 1) * sizeof(double)));
+        HIPCHECK(c, launch_loc_nlobsmax(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(),
+                                        c->d_glob.as<unsigned char>(), vis, c->d_nodes.as<KdNode>(),
+                                        c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt,
+                                        c->d_status.as<short>(), c->d_raw.as<int>(), c->d_rawoff.as<long long>(),
+                                        c->d_rrow.as<int>(), c->d_rd2.as<double>(), c->d_srow.as<int>(),
+                                        c->d_sd2.as<double>(), c->d_counts.as<int>()));
         HIPCHECK(c, launch_scan_counts(c->stream, c->d_counts.as<int>(), c->d_offsets.as<long long>(), ncnt,
                                        c->d_scantmp.p, &tmpb));
         HIPCHECK(c, hipMemcpyAsync(&total, c->d_offsets.as<long long>() + ncnt, sizeof total, hipMemcpyDeviceToHost,
@@ -634,15 +644,11 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
     // the Gram kernels read up to kListPad entries past the last list
     HIPCHECK(c, c->d_ids.reserve((total + kListPad) * sizeof(int)));
     HIPCHECK(c, c->d_lc.reserve((total + kListPad) * sizeof(double)));
-    c->lists_ordered = ordered || !boxes;
+    c->lists_ordered = ordered || nlobsmax;
     if (c->lists_ordered)
         HIPCHECK(c, fill_ordered(c, nlobsmax));
     else
-        HIPCHECK(c, launch_loc_box(c->stream, c->ni_s, c->nj_s, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
-                                   vis, c->d_types.as<TypeInfo>(), nt, c->d_boxes.as<LocBox>(), c->d_xyz.as<double>(),
-                                   c->nsearch, c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_counts.as<int>(),
-                                   c->d_lflag.as<int>(), c->d_offsets.as<long long>(), c->d_ids.as<int>(),
-                                   c->d_lc.as<double>()));
+        HIPCHECK(c, box(true));
     HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->timings[0] = elapsed(c->ev[0], c->ev[1]);
@@ -736,7 +742,7 @@ void enkfg_destroy(enkfg_ctx* c)
         (void)hipStreamSynchronize(c->stream2);
     DevBuf* bufs[] = {&c->d_nodes, &c->d_types, &c->d_obsids, &c->d_type, &c->d_status, &c->d_estd, &c->d_sqrtrf,
                       &c->d_perm, &c->d_S, &c->d_s, &c->d_tmp, &c->d_tmp2, &c->d_qxyz, &c->d_glob, &c->d_vis, &c->d_counts, &c->d_offsets,
-                      &c->d_scantmp, &c->d_ids, &c->d_lc, &c->d_run_ids, &c->d_run_lc, &c->d_lflag, &c->d_noderow, &c->d_xyz, &c->d_boxes,
+                      &c->d_scantmp, &c->d_ids, &c->d_lc, &c->d_run_ids, &c->d_run_lc, &c->d_lflag, &c->d_noderow, &c->d_rownode, &c->d_xyz, &c->d_boxes,
                       &c->d_raw, &c->d_rawoff, &c->d_rrow, &c->d_rd2,
                       &c->d_srow, &c->d_sd2, &c->d_T, &c->d_w, &c->d_T64, &c->d_w64, &c->d_pnlobs,
                       &c->d_pdfs, &c->d_psrf, &c->d_gram, &c->d_order, &c->d_segord, &c->d_sts, &c->d_err, &c->d_E, &c->d_infl, &c->d_nlev,
@@ -821,7 +827,6 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
     std::vector<unsigned char> placed((size_t)nobs, 0);
     c->perm.clear();
     c->perm.reserve(nobs);
-    c->box_ok = true;
     c->tinfo.assign(nt, TypeInfo{});
     for (int t = 0; t < nt; ++t) {
         const enkfg_obstype& ot = c->types[t];
@@ -853,8 +858,6 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
                 ti.nids++;
                 if (!std::isfinite(x[0]))
                     continue;
-                if (!std::isfinite(x[1]) || !std::isfinite(x[2]))
-                    c->box_ok = false;
                 found.push_back(i);
                 xyz.insert(xyz.end(), x, x + 3);
             }

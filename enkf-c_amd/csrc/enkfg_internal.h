@@ -60,12 +60,14 @@ hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz
                                const unsigned char* visible, const KdNode* nodes, const int* noderow,
                                const TypeInfo* types, int ntypes, const short* status, const int* raw, const long long* rawoff, int* rrow, double* rd2,
                                int* srow, double* sd2, int* counts);
-// the box search: with ids == nullptr counts the lists (and sets *tieflag if an
-// observation lies at exactly a type's radius), else fills them
+// the box search: with ids == nullptr counts the lists, else fills them.
+// nodes (and the row -> node map): the trees, for observations a whole radius
+// away along an axis; without them *tieflag is set if there is any
 hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
                           const unsigned char* visible, const TypeInfo* types, int ntypes, const LocBox* boxes,
-                          const double* xyz, size_t nrow, const short* status, const int* obsids, int* counts,
-                          int* tieflag, const long long* offsets, int* ids, double* lc);
+                          const double* xyz, size_t nrow, const short* status, const int* obsids,
+                          const KdNode* nodes, const int* rownode, int* counts, int* tieflag,
+                          const long long* offsets, int* ids, double* lc);
 hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
                            const unsigned char* visible, const KdNode* nodes, const int* noderow,
                            const TypeInfo* types, int ntypes, const short* status, const int* obsids, const long long* offsets, int* ids,

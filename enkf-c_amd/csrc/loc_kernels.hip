@@ -13,7 +13,13 @@
 // contraction, and a box is skipped only when its distance, rounded in the
 // same order, exceeds the radius -- rounding is monotone, so no observation
 // of it can be within the radius -- so the set and the taper bits are the
-// tree search's.
+// tree search's.  By the same argument the tree search reaches every
+// observation within the radius whose distance along each axis is below the
+// radius.  One at exactly the radius along an axis may lie behind a split
+// that was pruned: where counting finds any, it is done again with the trees,
+// and these observations climb theirs (walk_reaches).  A non-finite second
+// coordinate is in no list, in the tree on no finite observation's far side,
+// and left out of the boxes' bounds.
 //
 // The tree search walks the reference's own kd-trees (sequential insertion,
 // obs_createkdtrees) in the preorder of _kd_findnodeswithinrange
@@ -23,10 +29,7 @@
 // whether the far child is still to be visited, which depends only on that
 // node and the query.  Its lists are in the reference's order, element for
 // element: enkfg_localise and enkfg_get_localobs return those.  It also
-// decides what the box search cannot: an observation at exactly the radius is
-// in the list only if no split on its path is pruned, non-finite coordinates
-// follow the comparisons of the walk, and NLOBSMAX keeps candidates at equal
-// distance in visiting order.
+// serves NLOBSMAX, which keeps candidates at equal distance in visiting order.
 //
 // What bounds them, on the 51x1500x1800 tile (300,000 nodes, four types,
 // 1.86G entries, 22 GB of lists): the tree walk by the traffic of its node
@@ -552,9 +555,33 @@ __device__ inline void wave_lds_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
+// Does the tree walk reach node v?  Every ancestor must have led to v's side:
+// its near one, or the far one if the range crosses the split (range_walk_nd).
+template <int ND>
+__device__ inline bool walk_reaches(const KdNode* __restrict__ tree, int v, double range, double q0, double q1, double q2)
+{
+    int depth = 0;
+    for (int p = (int)(tree[v].link & 0x7fffffffu) - 1; p >= 0; p = (int)(tree[p].link & 0x7fffffffu) - 1)
+        ++depth;
+    while (depth > 0) {
+        const int p = (int)(tree[v].link & 0x7fffffffu) - 1;
+        const KdNode nd = tree[p];
+        const int dir = --depth % ND;
+        const double cd = dir == 0 ? nd.x : ((ND == 2 || dir == 1) ? nd.y : nd.z);
+        const double qd = dir == 0 ? q0 : ((ND == 2 || dir == 1) ? q1 : q2);
+        const double dx = qd - cd;
+        const bool left = (nd.link & 0x80000000u) && v == p + 1;
+        if (left != (dx <= 0.0) && !(fabs(dx) < range))
+            return false;
+        v = p;
+    }
+    return true;
+}
+
 template <int ND, bool FILL>
 __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ boxes, const double* __restrict__ xyz,
-                                 size_t nrow, const short* __restrict__ status, const double* q, int* __restrict__ ids,
+                                 size_t nrow, const short* __restrict__ status, const KdNode* __restrict__ nodes,
+                                 const int* __restrict__ rownode, const double* q, int* __restrict__ ids,
                                  double* __restrict__ lc, double* sd, int* si, bool& tie)
 {
     const int lane = threadIdx.x & 63;
@@ -613,9 +640,17 @@ __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ 
                             d = z[u] - q2;
                             distsq += d * d;
                         }
-                        const bool in = row[u] < row1 && distsq <= r2;
-                        tie |= in && distsq == r2;
-                        const bool ok = in && st[u] == kStatusOK;
+                        bool ok = row[u] < row1 && distsq <= r2 && st[u] == kStatusOK;
+                        // at exactly the range, all of it along one axis: the
+                        // walk may have pruned it
+                        if (__ballot(ok && distsq == r2)) {
+                            const bool along = ok && (fabs(x[u] - q0) >= ti.range || fabs(y[u] - q1) >= ti.range ||
+                                                      (ND == 3 && fabs(z[u] - q2) >= ti.range));
+                            if (nodes == nullptr)
+                                tie |= along;
+                            else if (along)
+                                ok = walk_reaches<ND>(nodes + ti.node0, rownode[row[u]], ti.range, q0, q1, q2);
+                        }
                         const unsigned long long m = __ballot(ok);
                         if (!FILL) {
                             n += __popcll(m);
@@ -660,6 +695,7 @@ __global__ void __launch_bounds__(256) loc_box_kernel(int ni, int nj, const doub
                                                       const LocBox* __restrict__ boxes,
                                                       const double* __restrict__ xyz, size_t nrow,
                                                       const short* __restrict__ status, const int* __restrict__ obsids,
+                                                      const KdNode* __restrict__ nodes, const int* __restrict__ rownode,
                                                       int* __restrict__ counts, const long long* __restrict__ offsets,
                                                       int* __restrict__ ids, double* __restrict__ lc,
                                                       int* __restrict__ tieflag)
@@ -693,8 +729,9 @@ __global__ void __launch_bounds__(256) loc_box_kernel(int ni, int nj, const doub
             int* wsi = FILL ? si + wave * 128 : nullptr;
             int* wid = FILL ? ids + o : nullptr;
             double* wlc = FILL ? lc + o : nullptr;
-            n = ti.ndim == 3 ? box_search<3, FILL>(ti, boxes, xyz, nrow, status, q, wid, wlc, wsd, wsi, tie)
-                             : box_search<2, FILL>(ti, boxes, xyz, nrow, status, q, wid, wlc, wsd, wsi, tie);
+            n = ti.ndim == 3
+                    ? box_search<3, FILL>(ti, boxes, xyz, nrow, status, nodes, rownode, q, wid, wlc, wsd, wsi, tie)
+                    : box_search<2, FILL>(ti, boxes, xyz, nrow, status, nodes, rownode, q, wid, wlc, wsd, wsi, tie);
             if (!FILL && __ballot(tie) && lane == 0)
                 atomicExch(tieflag, 1);
         }
@@ -887,8 +924,9 @@ hipError_t launch_scan_counts(hipStream_t s, const int* counts, long long* offse
 
 hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
                           const unsigned char* visible, const TypeInfo* types, int ntypes, const LocBox* boxes,
-                          const double* xyz, size_t nrow, const short* status, const int* obsids, int* counts,
-                          int* tieflag, const long long* offsets, int* ids, double* lc)
+                          const double* xyz, size_t nrow, const short* status, const int* obsids,
+                          const KdNode* nodes, const int* rownode, int* counts, int* tieflag,
+                          const long long* offsets, int* ids, double* lc)
 {
     if ((long long)ni * nj * ntypes <= 0)
         return hipSuccess;
@@ -899,10 +937,10 @@ hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, con
         return hipErrorInvalidValue;
     if (ids == nullptr)
         hipLaunchKernelGGL(loc_box_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, ni, nj, qxyz, isglobal,
-                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, counts, offsets, ids, lc, tieflag);
+                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc, tieflag);
     else
         hipLaunchKernelGGL(loc_box_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, ni, nj, qxyz, isglobal,
-                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, counts, offsets, ids, lc, tieflag);
+                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc, tieflag);
     return hipGetLastError();
 }
 

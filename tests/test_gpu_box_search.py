@@ -4,8 +4,9 @@ the reference's order after the calc (enkfg_get_localobs walks the trees for
 it), and T and w of the calc, which used the box search's lists.
 
 Sizes sit at the edges of the boxes (64 rows a leaf, 64 boxes a level).  The
-integer grids put many observations at exactly the radius (3-4-5 triples),
-where the tree search alone decides; a non-finite latitude does too.
+integer grids put many observations at exactly the radius, 3-4-5 triples and
+along an axis, where the reference's search prunes some; a few observations
+have no latitude.
 """
 import numpy as np
 import pytest
@@ -69,21 +70,27 @@ def test_box_search_sizes(n):
     assert run_case(types, typ, lon, lat, status, status2, nlon, nlat, 1) > 0
 
 
+@pytest.mark.parametrize("order", ["random", "sorted"])
 @pytest.mark.parametrize("bad", [False, True])
-def test_box_search_ties_and_nonfinite(bad):
+def test_box_search_ties_and_nonfinite(bad, order):
     """An integer grid in plain coordinates and radius 5: observations at
-    exactly the radius; with `bad`, also observations without a latitude."""
-    print("case box search ties bad=%d" % bad, flush=True)
+    exactly the radius, some of which the reference's search prunes; with
+    `bad`, also observations without a latitude."""
+    print("case box search ties bad=%d order=%s" % (bad, order), flush=True)
     rng = np.random.default_rng(4)
     x, y = np.meshgrid(np.arange(40), np.arange(30))
     lon, lat = x.ravel().astype(np.float32), y.ravel().astype(np.float32)
-    o = rng.permutation(lon.size)
+    o = rng.permutation(lon.size) if order == "random" else np.lexsort((lat, lon))
     lon, lat = lon[o], lat[o]
     typ = (np.arange(lon.size) % 2).astype(np.int16)
     if bad:
         lat[[7, 300]] = np.nan
+        lat[[17, 400]] = np.inf, -np.inf
         lon[11] = np.nan
     st = np.zeros(lon.size, np.int16)
     types = [dict(locrad=[5.0], geographic=0), dict(locrad=[4.5], geographic=0)]
     nlon, nlat = np.meshgrid(np.arange(1.0, 40.0, 6.0), np.arange(2.0, 30.0, 7.0))
-    assert run_case(types, typ, lon, lat, st, st, nlon, nlat, 0) > 0
+    found = run_case(types, typ, lon, lat, st, st, nlon, nlat, 0)
+    r = np.where(typ == 0, 5.0, 4.5)
+    near = ((lon[None] - nlon.ravel()[:, None]) ** 2 + (lat[None] - nlat.ravel()[:, None]) ** 2 <= r ** 2).sum()
+    assert 0 < found < near, "some observations at the radius are behind a pruned split"
