@@ -43,6 +43,8 @@
 //
 // The obs indices in the lists are device rows; the host maps them back to
 // observation indices.
+#include <algorithm>
+
 #include "enkfg_internal.h"
 
 namespace enkfg {
@@ -698,13 +700,13 @@ __global__ void __launch_bounds__(256) loc_box_kernel(int ni, int nj, const doub
                                                       const KdNode* __restrict__ nodes, const int* __restrict__ rownode,
                                                       int* __restrict__ counts, const long long* __restrict__ offsets,
                                                       int* __restrict__ ids, double* __restrict__ lc,
-                                                      int* __restrict__ tieflag)
+                                                      int* __restrict__ tieflag, unsigned run0)
 {
     __shared__ double sd[FILL ? 4 * 128 : 1];
     __shared__ int si[FILL ? 4 * 128 : 1];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned s = blockIdx.x / 8, x = blockIdx.x % 8;
-    const long long blk = ((long long)(s / kBoxRun) * 8 + x) * kBoxRun + s % kBoxRun;
+    const long long blk = ((long long)(run0 + s / kBoxRun) * 8 + x) * kBoxRun + s % kBoxRun;
     int t, node;
     if (!box_item(blk * 4 + wave, ni, nj, ntypes, t, node))
         return;
@@ -932,15 +934,22 @@ hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, con
         return hipSuccess;
     const long long blocks = (long long)((ni + 7) / 8) * ((nj + 7) / 8) * 16 * ntypes;
     const long long round = 8LL * kBoxRun;
-    const long long grid = round * ((blocks + round - 1) / round);
-    if (grid > 0x7fffffffLL)
+    const long long rounds = (blocks + round - 1) / round;
+    if (rounds > 0xffffffffLL)
         return hipErrorInvalidValue;
-    if (ids == nullptr)
-        hipLaunchKernelGGL(loc_box_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, ni, nj, qxyz, isglobal,
-                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc, tieflag);
-    else
-        hipLaunchKernelGGL(loc_box_kernel<true>, dim3((unsigned)grid), dim3(256), 0, s, ni, nj, qxyz, isglobal,
-                           visible, types, ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc, tieflag);
+    // a launch holds fewer than 2^32 threads: 16M blocks, 64M lists
+    constexpr long long per = (1LL << 24) / (8 * kBoxRun) - 1;
+    for (long long r0 = 0; r0 < rounds; r0 += per) {
+        const dim3 grid((unsigned)(round * std::min(per, rounds - r0)));
+        if (ids == nullptr)
+            hipLaunchKernelGGL(loc_box_kernel<false>, grid, dim3(256), 0, s, ni, nj, qxyz, isglobal, visible, types,
+                               ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc,
+                               tieflag, (unsigned)r0);
+        else
+            hipLaunchKernelGGL(loc_box_kernel<true>, grid, dim3(256), 0, s, ni, nj, qxyz, isglobal, visible, types,
+                               ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc,
+                               tieflag, (unsigned)r0);
+    }
     return hipGetLastError();
 }
 

@@ -94,3 +94,42 @@ def test_box_search_ties_and_nonfinite(bad, order):
     r = np.where(typ == 0, 5.0, 4.5)
     near = ((lon[None] - nlon.ravel()[:, None]) ** 2 + (lat[None] - nlat.ravel()[:, None]) ** 2 <= r ** 2).sum()
     assert 0 < found < near, "some observations at the radius are behind a pruned split"
+
+
+def test_box_search_beyond_one_launch():
+    """8.45M nodes and 8 types: more lists (67.6M) than one launch has
+    wavefronts for (2^32 threads).  A few observations of each type on planar
+    coordinates, at the corners and the middle; every count of the calc (EnOI,
+    two members), and lists at the end of the grid."""
+    print("case box search beyond one launch", flush=True)
+    ni, nj, nt, r = 8192, 1032, 8, 2.5
+    rng = np.random.default_rng(8)
+    base = np.array([[0.3, 0.4], [8190.2, 0.7], [0.1, 1030.4], [8190.6, 1030.8], [4000.3, 515.2], [8188.9, 1029.7]])
+    xy = np.concatenate([base + 0.1 * rng.random(base.shape) for _ in range(nt)]).astype(np.float32)
+    typ = np.repeat(np.arange(nt, dtype=np.int16), len(base))
+    n = len(typ)
+    types = [dict(locrad=[r], geographic=0) for _ in range(nt)]
+    estd = np.full(n, 0.5, np.float32)
+    st = np.zeros(n, np.int16)
+    E = enkfg.Engine(2, mode=enkfg.MODE_ENOI)
+    E.set_obstypes(types)
+    E.set_obs(typ, st, xy[:, 0], xy[:, 1], estd)
+    E.set_S(rng.standard_normal((2, n)).astype(np.float32), rng.standard_normal(n), standardised=False)
+    nlon, nlat = np.meshgrid(np.arange(float(ni)), np.arange(float(nj)))
+    E.calc_transforms(nlon, nlat, geographic=0)
+    pn, _, _ = E.diag()
+    want = np.zeros((nt + 1, nj, ni), np.int32)
+    for (x, y), t in zip(xy.astype(np.float64), typ):
+        i0, j0 = max(int(x) - 4, 0), max(int(y) - 4, 0)
+        w = (slice(j0, j0 + 9), slice(i0, i0 + 9))
+        hit = (nlon[w] - x) ** 2 + (nlat[w] - y) ** 2 <= r * r
+        for q in (t, nt):
+            want[q][w] += hit
+    assert want[:nt].any(axis=(1, 2)).all()
+    assert np.array_equal(pn.reshape(want.shape), want)
+    ob = O.OracleObs(types, typ, xy[:, 0], xy[:, 1], estd)
+    for k in (0, ni - 1, ni * nj - 1, ni * nj - 2, ni * (nj - 2) + 8190):
+        ids, lc = ob.findlocal(nlon.ravel()[k], nlat.ravel()[k], 0)
+        got = E.localobs(k, n)
+        assert len(ids) and np.array_equal(got[0][:len(ids)], ids) and np.array_equal(got[1][:len(ids)], lc)
+    E.close()
