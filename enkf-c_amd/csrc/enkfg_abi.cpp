@@ -393,6 +393,9 @@ int node_inputs(enkfg_ctx* c, const enkfg_nodes* nodes)
     const long long nn = (long long)nodes->ni * nodes->nj;
     if (nn > 0x7fffffffLL)
         return fail(c, ENKFG_ERR_ARG, "too many nodes");
+    c->lists_valid = false;   // (a call refused above leaves the lists)
+    c->run_n = 0;
+    c->run_next = kOrderRun;
     c->nnode = (int)nn;
     c->ni_s = nodes->ni;
     c->nj_s = nodes->nj;
@@ -556,9 +559,6 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
     for (const auto& t : c->types)
         if (t.nlobsmax != ENKFG_NLOBSMAX_NONE)
             nlobsmax = true;
-    c->lists_valid = false;
-    c->run_n = 0;
-    c->run_next = kOrderRun;
     int r = node_inputs(c, nodes);
     if (r != ENKFG_OK)
         return r;
@@ -820,7 +820,8 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
     // curve, then every other obs.  64 consecutive rows of a type share a box,
     // 64 boxes one of the next level.
     c->trees_built = false;
-    c->obs_set = false;
+    // (nothing of the old obs is used should one of the steps below fail)
+    c->obs_set = c->S_set = c->lists_valid = false;
     std::vector<int> obsids;
     std::vector<double> coords;   // [row][3]
     std::vector<LocBox> boxes;
@@ -951,8 +952,6 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
     HIPCHECK(c, c->d_sqrtrf.reserve(srf.size() * sizeof(double)));
     HIPCHECK(c, hipMemcpy(c->d_sqrtrf.p, srf.data(), srf.size() * sizeof(double), hipMemcpyHostToDevice));
     c->obs_set = true;
-    c->S_set = false;
-    c->lists_valid = false;
     return ENKFG_OK;
 }
 

@@ -1,5 +1,7 @@
 """The local lists between calls, through the C ABI: which node grid they
 belong to, what reads them, and what leaves them as they are."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -86,4 +88,20 @@ def test_lists_read_across_runs():
     lon[0, 7] = lon[30, 5] = lon[36, 52] = np.nan
     E.calc_transforms(lon, lat, stride=P.stride)
     check_lists(E, ob, lon, lat, [1960, 0, 7, 1023, 1024, 1025, 1599, 63, 64, 1959, 1952, 1951, 1023, 1595, 1960])
+    E.close()
+
+
+def test_a_refused_call_leaves_the_lists():
+    """A node grid that is refused (no nodes, no coordinates), by the calc or
+    the localisation, leaves the lists of the calc before it."""
+    print("case refused node grids", flush=True)
+    P, E, ob = setup()
+    E.calc_transforms(P.node_lon, P.node_lat, stride=P.stride)
+    lon = P.node_lon.ctypes.data_as(C.POINTER(C.c_double))
+    for call in (enkfg.lib().enkfg_calc_transforms, enkfg.lib().enkfg_localise):
+        for nd in (enkfg.Nodes(0, 5, 1, 1, lon, lon, None), enkfg.Nodes(2, 2, 1, 1, lon, None, None)):
+            assert call(E.h, C.byref(nd)) != 0
+            check_lists(E, ob, P.node_lon, P.node_lat, [0, 17])
+        assert call(E.h, None) != 0
+    assert len(E.local_counts()) == P.node_lon.size
     E.close()
