@@ -372,8 +372,7 @@ hipError_t launch_gram(hipStream_t s, const CalcArgs& a)
     // larger by default)
     const int lo = item_groups_lo(MT);
     const long long nlist = (long long)a.nbatch * a.nseg;
-    const int ng = nlist * item_groups_many(MT) <= kManyItems ? item_groups_many(MT)
-                                                              : (a.tile_groups == lo ? lo : lo + 1);
+    const int ng = few_lists(MT, nlist) ? item_groups_many(MT) : (a.tile_groups == lo ? lo : lo + 1);
     const long long nitem = (long long)a.nbatch * a.nseg * ng;
     const dim3 igrid(item_grid(nitem));
     switch (MT) {

@@ -1454,6 +1454,10 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
     const bool mixed = c->cfg.precision == ENKFG_PREC_MIXED;
     const bool items = (m + 15) / 16 <= 10;
     const int kTuneMin = std::min(nbatch, 256);
+    // (a launch of few lists takes a group count of its own: the candidates
+    // would be the same kernel)
+    const auto few = [&](int n) { return few_lists((m + 15) / 16, (long long)n * nseg); };
+    const auto tunable = [&](int n) { return items && n >= kTuneMin && !few(n); };
     int* tg = c->tile_groups[mixed ? 1 : 0];
     const int tg_lo = item_groups_lo((m + 15) / 16);
     const int tg_default = mixed ? tg_lo : tg_lo + 1;
@@ -1464,7 +1468,7 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
         for (int q = 0; q < kBuckets; ++q) {
             if (bcount[q] == 0)
                 continue;
-            if (tg[q] == 0 && bcount[q] >= kTuneMin)
+            if (tg[q] == 0 && tunable(std::min(nbatch, bcount[q])))
                 tuned = false;
             const int g = tg[q] ? tg[q] : tg_default;
             if (common == 0)
@@ -1472,7 +1476,7 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
             else if (g != common)
                 same = false;
         }
-        plain = tuned && same;
+        plain = few(nn) || (tuned && same);
     }
     struct Batch {
         int node0, n, bucket;
@@ -1504,7 +1508,7 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
     // every buffer the kernels read or write -- is unchanged.
     bool need_tune = false;
     for (const Batch& bt : batches)
-        if (items && bt.bucket >= 0 && tg[bt.bucket] == 0 && bt.n >= kTuneMin)
+        if (bt.bucket >= 0 && tg[bt.bucket] == 0 && tunable(bt.n))
             need_tune = true;
     if ((c->cfg.flags & ENKFG_FLAG_GRAPH) && !need_tune && nb > 0) {
         std::vector<long long> sig = {nb, (long long)mixed, plain_groups, (long long)(intptr_t)a.node_list,
@@ -1613,7 +1617,7 @@ int enkfg_calc_transforms(enkfg_ctx* c, const enkfg_nodes* nodes)
         if (bk < 0) {
             a.tile_groups = plain_groups;
             HIPCHECK(c, mixed ? launch_gram_mixed(c->stream, a) : launch_gram(c->stream, a));
-        } else if (items && tg[bk] == 0 && a.nbatch >= kTuneMin) {
+        } else if (tg[bk] == 0 && tunable(a.nbatch)) {
             // the default shape first; the other is kept only when it is
             // clearly faster (3%), so that run-to-run noise does not flip
             // the choice

@@ -30,9 +30,11 @@ __host__ __device__ constexpr int item_groups_lo(int MT)
 // chunks take less time each and more wavefronts share the work (9 nodes of
 // four lists, the longest 3,000 obs, m = 96: 0.41 ms with two groups).  Used
 // where even then the items are fewer than kManyItems, two wavefronts per
-// SIMD; the matrices are the same bit for bit.
+// SIMD (few_lists), whatever CalcArgs::tile_groups asks for; such launches are
+// not tuned.  The matrices are the same bit for bit.
 __host__ __device__ constexpr int item_groups_many(int MT) { return MT <= 4 ? item_groups_lo(MT) + 1 : (tri_count(MT) + 2) / 3; }
 constexpr long long kManyItems = 2048;
+inline bool few_lists(int MT, long long nlist) { return nlist * item_groups_many(MT) <= kManyItems; }
 
 // The items (segment, tile group) of the item Gram kernels are dealt to the 8
 // XCDs in runs of kItemRun.  Block i runs on XCD i % 8 (the hardware

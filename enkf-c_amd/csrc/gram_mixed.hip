@@ -286,8 +286,7 @@ hipError_t launch_gram_mixed(hipStream_t s, const CalcArgs& a)
         // smaller by default)
         const int lo = item_groups_lo(MT);
         const long long nlist = (long long)a.nbatch * a.nseg;
-        const int ng = nlist * item_groups_many(MT) <= kManyItems ? item_groups_many(MT)
-                                                                  : (a.tile_groups == lo + 1 ? lo + 1 : lo);
+        const int ng = few_lists(MT, nlist) ? item_groups_many(MT) : (a.tile_groups == lo + 1 ? lo + 1 : lo);
         const long long nitem = (long long)a.nbatch * a.nseg * ng;
         const dim3 igrid(item_grid(nitem));
         switch (MT) {

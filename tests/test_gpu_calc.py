@@ -358,3 +358,36 @@ def test_calc_empty_columns_and_stats():
     assert not w[empty].any()
     assert E.stats() == ref["stats"]
     E.close()
+
+
+@pytest.mark.parametrize("precision", [enkfg.PREC_FP64, enkfg.PREC_MIXED])
+def test_few_columns_are_not_tuned(precision):
+    """The launches of a few columns take a tile group count of their own, so
+    a calc on nine columns leaves the tuning open; the next large calc of the
+    engine tunes its buckets, and its results are those of a fresh engine."""
+    print("case few columns precision=%d" % precision, flush=True)
+    P = problem(seed=12, nmem=24, nobs=2500, locrad=75.0, nj=45, ni=60, stride=1)
+
+    def engine():
+        E = enkfg.Engine(24, precision=precision)
+        E.set_obstypes(P.obstypes)
+        E.set_obs(P.obs_type, P.obs_status, P.obs_lon, P.obs_lat, P.obs_estd)
+        E.set_S(P.HA, P.innov, standardised=False)
+        return E
+
+    key = "groups_fp64" if precision == enkfg.PREC_FP64 else "groups_mixed"
+    E = engine()
+    for _ in range(2):
+        E.calc_transforms(P.node_lon[20:23, 30:33].copy(), P.node_lat[20:23, 30:33].copy())
+        assert sum(b["nodes"] for b in E.tuning()) == 9 and not any(b[key] for b in E.tuning())
+        assert E.launches() == 1
+    E.calc_transforms(P.node_lon, P.node_lat)
+    big = [b for b in E.tuning() if b["nodes"] >= 1024]
+    assert big and all(b[key] for b in big)
+    T, w, _, _ = E.transforms()
+    F = engine()
+    F.calc_transforms(P.node_lon, P.node_lat)
+    T2, w2, _, _ = F.transforms()
+    assert np.array_equal(T, T2) and np.array_equal(w, w2)
+    E.close()
+    F.close()
