@@ -120,6 +120,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
             const bool first = ph == 0;
             const bool ofY = first || (ph & 1) != 0;   // the inverse goes into Z
             tile4 x[tri_count(MT)];
+            // diagonal tiles are read as other lanes of this wavefront stored them
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             read_tiles<MT, 0, tri_count(MT)>(ofY ? Y : Z, lane, x);
 #pragma unroll
             for (int f = 0; f < tri_count(MT); ++f)
