@@ -439,6 +439,15 @@ def test_adjoint_ens_against_autograd(mode, m, md, alpha):
     assert np.abs(gR_ref).max() > 0 and gi_ref[1] != 0.0
 
 
+@pytest.mark.parametrize("mode,m,md", [(enkfg.MODE_ENKF, m, m) for m in (5, 15, 16, 17, 33, 47, 64, 65, 81, 95)]
+                         + [(enkfg.MODE_HYBRID, 49, 31)])
+def test_adjoint_ens_member_counts(mode, m, md):
+    """The same at the edges of the kernels' 16-member tiles, and member
+    counts that are odd."""
+    test_adjoint_ens_against_autograd(mode, m, md, 0.9)
+
+
+
 def test_adjoint_ens_c5_m96_against_autograd_and_finite_differences():
     """enkfg_adjoint_ens at the C5 size: 32 layers x 600 x 600, m = 96, 1M
     surface obs, LOCRAD 200 km, stride 3, DEnKF, capped inflation 1.05 (ratio

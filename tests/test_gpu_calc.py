@@ -75,15 +75,12 @@ def test_localisation_status_visibility_global():
     E.close()
 
 
-def test_localisation_one_walk_and_pool_overflow():
-    """Localisations after the first walk the trees once, into a pool of
-    chunks sized by the previous lists, and compact them; a pool too small
-    for the new lists falls back to counting first.  Three localisations of
-    one engine: type 1 invisible (two walks), all visible with a global node
-    (the pool overflows: two walks again), and the same again (one walk,
-    with the global node's list written by the compaction) -- each against
-    the oracle, bit for bit."""
-    print("case localisation one walk / pool overflow", flush=True)
+def test_localisation_repeated_with_other_types_visible():
+    """Three localisations and calcs of one engine: type 1 invisible, all
+    visible, and the same again, with a global node -- each against the oracle,
+    bit for bit.  enkfg_localise walks the trees; the calc searches the boxes,
+    and its lists are read in the reference's order."""
+    print("case localisation repeated, visibility", flush=True)
     P = problem(seed=7, profiles=30, nobs=3000, locrad=90.0)
     rng = np.random.default_rng(11)
     status = P.obs_status.copy()
@@ -94,16 +91,18 @@ def test_localisation_one_walk_and_pool_overflow():
     lon = P.node_lon.copy()
     lat = P.node_lat.copy()
     lon[1, 2] = np.nan                              # a node without coordinates -> all obs of each type
+    E.set_S(P.HA, P.innov, standardised=False)
     for vis in (np.array([1, 0], np.uint8), np.array([1, 1], np.uint8), np.array([1, 1], np.uint8)):
-        E.localise(lon, lat, stride=P.stride, visible=vis)
-        counts = E.local_counts()
-        assert counts.sum() > 0
-        for k in range(lon.size):
-            ids_o, lc_o = ob.findlocal(lon.flat[k], lat.flat[k], visible=vis)
-            assert counts[k] == len(ids_o), "node %d count" % k
-            ids_g, lc_g = E.localobs(k, counts[k])
-            assert np.array_equal(ids_g[:counts[k]], ids_o), "node %d ids" % k
-            assert np.array_equal(lc_g[:counts[k]].view(np.uint64), lc_o.view(np.uint64))
+        for call in (E.localise, E.calc_transforms):
+            call(lon, lat, stride=P.stride, visible=vis)
+            counts = E.local_counts()
+            assert counts.sum() > 0
+            for k in range(lon.size):
+                ids_o, lc_o = ob.findlocal(lon.flat[k], lat.flat[k], visible=vis)
+                assert counts[k] == len(ids_o), "node %d count" % k
+                ids_g, lc_g = E.localobs(k, counts[k])
+                assert np.array_equal(ids_g[:counts[k]], ids_o), "node %d ids" % k
+                assert np.array_equal(lc_g[:counts[k]].view(np.uint64), lc_o.view(np.uint64))
     E.close()
 
 
@@ -111,8 +110,8 @@ def test_localisation_one_walk_and_pool_overflow():
                                             (enkfg.PREC_FP64, 144), (enkfg.PREC_MIXED, 144)])
 def test_calc_buckets_and_autotune_bitwise(precision, nmem):
     """The calc orders the nodes by obs-count bucket and tunes each bucket's
-    Gram tile groups (wavefronts per list: 2 or 3 for m <= 96, 4 or 5 for
-    m = 144) on its first large batch, running both.  A node's Gram matrix
+    Gram tile groups (wavefronts per list: 2 or 3 for the 24 members here, 4
+    or 5 for m = 144) on its first large batch, running both.  A node's Gram matrix
     does not depend on the order or the tile groups, so a second calc on the
     same engine (tuned choices) gives T, w and the diagnostics of the first
     (tuning) calc bit for bit; the buckets account for every node."""
