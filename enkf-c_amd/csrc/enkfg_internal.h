@@ -139,7 +139,8 @@ struct CalcArgs {
     // ceil(m / 16), zero outside m x m) for the adjoint through T
     double* adj_minv;
     // Gram item kernels: tile groups (wavefronts) per segment, item_groups_lo or
-    // one more; any other value takes the default (one more FP64, lo mixed)
+    // one more; any other value takes the default (one more FP64, lo mixed).
+    // Launches of few lists (few_lists) take item_groups_many instead.
     int tile_groups;
     // ETKF: workspace of etkf_groups(m, nbatch) wavefronts, etkf_ws_size(m)
     // doubles each

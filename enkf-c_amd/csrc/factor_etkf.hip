@@ -27,7 +27,9 @@
 // workgroup barrier, one five-wave workgroup per CU): 51x1500x1800 tile FP64
 // calc 1,909 -> 561 ms; 4,050 nodes, m = 96: 21.0 -> 4.3 ms; 2,278 nodes, m =
 // 24: 0.61 -> 0.22 ms.  m > 96 had iterates in memory and Gauss-Jordan
-// inverses of up to 2 KB of spills a lane; it takes the same path now.
+// inverses of up to 2 KB of spills a lane; it takes the same path now (488
+// and 980 B of spills at MT = 9 and 10, 164 at 6: tile_waves).  Counters on the
+// tile: matrix cores busy 41%, VALU issue 26%.
 #include <algorithm>
 
 #include "enkfg_internal.h"

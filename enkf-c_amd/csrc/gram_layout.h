@@ -9,18 +9,22 @@
 namespace enkfg {
 
 // Upper-triangular 16x16 tiles (I <= J) of an MT x MT tile grid, enumerated
-// row by row; wave w of the 4 waves of a Gram workgroup owns tiles w, w + 4,
-// w + 8, ...
+// row by row
 __host__ __device__ constexpr int tri_count(int MT) { return MT * (MT + 1) / 2; }
 
-// The item Gram kernels split a segment's tri_count(MT) tiles into NG groups,
-// one wavefront each; the two candidates per MT are lo and lo + 1, lo chosen
-// so that a group's accumulators and operands fit the 256 registers of a
-// lane (m = 96: all 21 tiles in one wavefront, 244 registers, so that each
-// observation is read and converted once: FP64 calc on the 51x1500x1800 tile
-// 379 ms against 412 for two groups of unpipelined k-steps; 28 tiles: 3 or 4
-// groups; 36 and 45: 4 or 5; 55: 5 or 6).  Up to m = 64 a segment has ten
-// tiles or fewer and two wavefronts are kept, for launches of few nodes.
+// The item Gram kernels split a segment's tri_count(MT) tiles into NG groups
+// (group g: tiles g, g + NG, ...), one wavefront each; the two candidates per MT
+// are lo and lo + 1.  An observation is read and converted once per group, so
+// fewer groups do less work, as far as a group's accumulators and operands
+// fit the 256 registers of a lane beside two wavefronts a SIMD.  m = 96: all
+// 21 tiles in one wavefront take 244 registers (mixed 217); FP64 calc on the
+// 51x1500x1800 tile 379 ms against 412 for two groups of unpipelined k-steps.
+// Up to m = 64 a segment has ten tiles or fewer and two wavefronts are kept,
+// for launches of few nodes.  From MT = 7 on the counts (3, 4, 4, 5) are those
+// that were measured with the kernels before the pipelined k-steps (156 to 193
+// registers, mixed 180 to 228); 2, 2, 3 and 4 would fit too, with 193, 234, 215
+// and 214 registers (mixed 205, 238, 230, 247) and no vector spills, and have
+// not been measured.
 __host__ __device__ constexpr int item_groups_lo(int MT)
 {
     return MT <= 4 ? 2 : (MT <= 6 ? 1 : (MT == 7 ? 3 : (MT <= 9 ? 4 : 5)));
@@ -111,14 +115,5 @@ __host__ __device__ constexpr int tri_J(int MT, int f)
 // kernel stores and the factor kernels load whole 512-byte runs (and 21
 // tiles instead of 36 for m = 96).
 __host__ __device__ constexpr size_t gram_size(int MT) { return (size_t)tri_count(MT) * 256; }
-
-// position of element (i, j) of the symmetric matrix
-__host__ __device__ constexpr size_t gram_at(int MT, int i, int j)
-{
-    const int I = i / 16, J = j / 16;
-    if (I > J || (I == J && i > j))
-        return gram_at(MT, j, i);
-    return ((size_t)(I * MT - I * (I - 1) / 2 + (J - I)) * 16 + i % 16) * 16 + j % 16;
-}
 
 }  // namespace enkfg

@@ -6,9 +6,9 @@
 // hi = bf16(x), lo = bf16(x - hi) and |r| <= 2^-18 |x|; the product x_a x_b
 // is taken as hi_a hi_b + hi_a lo_b + lo_a hi_b, which leaves out lo_a lo_b
 // (<= 2^-18 relative), so every term of S^T S carries a relative error of
-// about 2^-17 before the FP32 accumulation.  S^T s accumulates in FP64 from
-// x.  The result is written in the FP64 Gram layout and the
-// factorisation that follows stays in FP64 (factor_tile.hip).
+// about 2^-17 before the FP32 accumulation.  S^T s is summed from x, in FP32
+// over four obs and in FP64 beyond.  The result is written in the FP64 Gram
+// layout and the factorisation that follows stays in FP64 (factor_tile.hip).
 //
 // Work items, chunk pipeline and XCD placement are those of the FP64 item
 // Gram kernel (calc_kernels.hip, gram_stage.h, gram_layout.h).

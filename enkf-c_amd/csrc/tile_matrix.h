@@ -284,8 +284,13 @@ __device__ __attribute__((always_inline)) inline void tile_inverse(const tile4* 
     });
 }
 
-// wavefronts per SIMD that the tiles' registers allow (8 per tile, and about
-// 60 beside them)
+// wavefronts per SIMD for which the kernels are compiled: a lane's share of a
+// SIMD's 512 registers is 8 for each tile and what the kernel needs beside
+// them, which is more than the rest of the share for some MT: the DEnKF and
+// trace kernels spill 10 and 8 registers at MT = 6, 14 and 8 at 8, 206 and 130
+// at 9, 789 and 542 at 10, the ETKF kernel 24, 97, 97, 22, 32, 291 and 956 at
+// 2, 3, 6, 7, 8, 9 and 10 (compiler's report).  Other counts for these have
+// not been measured.
 __host__ __device__ constexpr int tile_waves(int MT) { return MT <= 3 ? 4 : (MT <= 6 ? 2 : 1); }
 
 constexpr double kDfsMin = 1.0e-6;   // DFS_MIN, calc/transforms.c:32

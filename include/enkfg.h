@@ -232,7 +232,11 @@ int enkfg_get_diag(enkfg_ctx* ctx, int* pnlobs, float* pdfs, float* psrf);
 int enkfg_get_stats(enkfg_ctx* ctx, enkfg_stats* stats);
 
 /* Localisation only (obs_findlocal for every node); lists are kept on the
- * device.  counts: [node]; a node's list is read with enkfg_get_localobs. */
+ * device.  counts: [node]; a node's list is read with enkfg_get_localobs, in
+ * the reference's order.  That order is that of the reference's kd-trees,
+ * which the calc does without: they are built on the host by the first
+ * enkfg_localise after enkfg_set_obs, or the first enkfg_get_localobs after a
+ * calc, which then also walks them for the node and its neighbours. */
 int enkfg_localise(enkfg_ctx* ctx, const enkfg_nodes* nodes);
 int enkfg_get_local_counts(enkfg_ctx* ctx, int* counts);
 int enkfg_get_localobs(enkfg_ctx* ctx, int node, int cap, int* ids, double* lc);
@@ -369,11 +373,13 @@ int enkfg_get_timings(enkfg_ctx* ctx, double* ms, int n);
  * obs-count bucket (the largest (node, obstype) list: [0, 256), [256, 1024),
  * [1024, 4096), [4096, ...)), heaviest bucket first, and runs each bucket's
  * Gram matrices with the tile groups per list (wavefronts: 2 or 3 for
- * nmem <= 64, 1 or 2 up to 96, 3 or 4 up to 112, 4 or 5 up to 144, 5 or 6 up to 160) that the
- * first sufficiently large batch of the bucket measured fastest.  Writes up
- * to n ints: out[0] = number of buckets B, then per bucket the lower bound,
- * the nodes in it at the last calc, and the tile groups chosen for FP64 and
- * for mixed precision (0 = not tuned yet). */
+ * nmem <= 64, 1 or 2 up to 96, 3 or 4 up to 112, 4 or 5 up to 144, 5 or 6 up
+ * to 160) that the first sufficiently large batch of the bucket measured
+ * fastest.  A calc, or batch, of few lists runs in one shape of its own, with
+ * more groups, and chooses nothing.  Writes up to n ints: out[0] = number of
+ * buckets B, then per bucket the lower bound, the nodes in it at the last
+ * calc, and the tile groups chosen for FP64 and for mixed precision (0 = not
+ * tuned yet). */
 int enkfg_get_tuning(enkfg_ctx* ctx, int* out, int n);
 
 #ifdef __cplusplus
