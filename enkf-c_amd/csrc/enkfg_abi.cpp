@@ -120,6 +120,7 @@ struct enkfg_ctx {
     std::vector<int> perm;
     size_t nsearch = 0;           // rows that are searched (the types' rows come first)
     bool trees_built = false;     // d_nodes, d_noderow, d_rownode hold the reference's trees
+    bool ties = false;            // a search has met an obs a whole radius away along an axis
 
     // S and s
     DevBuf d_S, d_s, d_tmp, d_tmp2;
@@ -583,7 +584,7 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
     HIPCHECK(c, hipEventRecord(c->ev[0], c->stream));
     long long total = 0;
     const auto box = [&](bool fill) {
-        const bool trees = c->trees_built;
+        const bool trees = c->ties;
         return launch_loc_box(c->stream, c->list_ni, c->list_nj, c->d_qxyz.as<double>(),
                               c->d_glob.as<unsigned char>(), vis, c->d_types.as<TypeInfo>(), nt,
                               c->d_boxes.as<LocBox>(), c->d_xyz.as<double>(), c->nsearch, c->d_status.as<short>(),
@@ -592,8 +593,8 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
                               c->d_offsets.as<long long>(), fill ? c->d_ids.as<int>() : nullptr,
                               fill ? c->d_lc.as<double>() : nullptr);
     };
-    for (int tie = nlobsmax ? 0 : 1; tie != 0;) {   // again with the trees if there are ties
-        const bool trees = c->trees_built;
+    for (bool counted = nlobsmax; !counted;) {   // again with the trees if there are ties
+        int tie = 0;
         HIPCHECK(c, hipMemsetAsync(c->d_lflag.p, 0, sizeof(int), c->stream));
         HIPCHECK(c, box(false));
         HIPCHECK(c, launch_scan_counts(c->stream, c->d_counts.as<int>(), c->d_offsets.as<long long>(), ncnt,
@@ -602,12 +603,12 @@ int do_localise(enkfg_ctx* c, const enkfg_nodes* nodes, bool ordered)
                                    c->stream));
         HIPCHECK(c, hipMemcpyAsync(&tie, c->d_lflag.p, sizeof tie, hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
-        if (trees)
-            break;
+        counted = c->ties || tie == 0;
         if (tie != 0) {
             r = ensure_trees(c);
             if (r != ENKFG_OK)
                 return r;
+            c->ties = true;
         }
     }
     if (nlobsmax) {
@@ -819,7 +820,7 @@ int enkfg_set_obs(enkfg_ctx* c, int nobs, const short* type, const short* status
     // status OK, finite first coordinate (kd_insertnode) -- along a Morton
     // curve, then every other obs.  64 consecutive rows of a type share a box,
     // 64 boxes one of the next level.
-    c->trees_built = false;
+    c->trees_built = c->ties = false;
     // (nothing of the old obs is used should one of the steps below fail)
     c->obs_set = c->S_set = c->lists_valid = false;
     std::vector<int> obsids;

@@ -62,7 +62,8 @@ hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz
                                int* srow, double* sd2, int* counts);
 // the box search: with ids == nullptr counts the lists, else fills them.
 // nodes (and the row -> node map): the trees, for observations a whole radius
-// away along an axis; without them *tieflag is set if there is any
+// away along an axis; counting without them sets *tieflag if there is any, and
+// the lists are then to be counted and filled with them
 hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
                           const unsigned char* visible, const TypeInfo* types, int ntypes, const LocBox* boxes,
                           const double* xyz, size_t nrow, const short* status, const int* obsids,

@@ -580,7 +580,9 @@ __device__ inline bool walk_reaches(const KdNode* __restrict__ tree, int v, doub
     return true;
 }
 
-template <int ND, bool FILL>
+// TREES: observations a whole range away along an axis climb their tree; else
+// counting sets tie for them (and there are none when the lists are filled)
+template <int ND, bool FILL, bool TREES>
 __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ boxes, const double* __restrict__ xyz,
                                  size_t nrow, const short* __restrict__ status, const KdNode* __restrict__ nodes,
                                  const int* __restrict__ rownode, const double* q, int* __restrict__ ids,
@@ -630,8 +632,9 @@ __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ 
                         z[u] = ND == 3 ? Z[r] : 0.0;
                         st[u] = status[r];
                     }
-#pragma unroll
-                    for (int u = 0; u < kBoxAhead; ++u) {
+                    double dsq[kBoxAhead];
+                    bool ok[kBoxAhead], at = false;
+                    const auto test = [&](int u) {
                         // kd_findnodeswithinrange's sum, in its order (kdtree.c:529-533)
                         double distsq = 0.0;
                         double d = x[u] - q0;
@@ -642,24 +645,18 @@ __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ 
                             d = z[u] - q2;
                             distsq += d * d;
                         }
-                        bool ok = row[u] < row1 && distsq <= r2 && st[u] == kStatusOK;
-                        // at exactly the range, all of it along one axis: the
-                        // walk may have pruned it
-                        if (__ballot(ok && distsq == r2)) {
-                            const bool along = ok && (fabs(x[u] - q0) >= ti.range || fabs(y[u] - q1) >= ti.range ||
-                                                      (ND == 3 && fabs(z[u] - q2) >= ti.range));
-                            if (nodes == nullptr)
-                                tie |= along;
-                            else if (along)
-                                ok = walk_reaches<ND>(nodes + ti.node0, rownode[row[u]], ti.range, q0, q1, q2);
-                        }
-                        const unsigned long long m = __ballot(ok);
+                        dsq[u] = distsq;
+                        ok[u] = row[u] < row1 && distsq <= r2 && st[u] == kStatusOK;
+                        at |= ok[u] && distsq == r2;
+                    };
+                    const auto put = [&](int u) {
+                        const unsigned long long m = __ballot(ok[u]);
                         if (!FILL) {
                             n += __popcll(m);
                         } else if (m) {
-                            if (ok) {
+                            if (ok[u]) {
                                 const int pos = nbuf + __popcll(m & below);
-                                sd[pos] = distsq;
+                                sd[pos] = dsq[u];
                                 si[pos] = row[u];
                             }
                             nbuf += __popcll(m);
@@ -677,7 +674,48 @@ __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ 
                                 wave_lds_fence();
                             }
                         }
+                    };
+                    if (FILL && !TREES) {
+#pragma unroll
+                        for (int u = 0; u < kBoxAhead; ++u) {
+                            test(u);
+                            put(u);
+                        }
+                        continue;
                     }
+#pragma unroll
+                    for (int u = 0; u < kBoxAhead; ++u)
+                        test(u);
+                    if (__builtin_expect(__ballot(at) != 0, 0)) {
+                        // at exactly the range: where all of it is along one
+                        // axis the walk may have pruned it
+                        unsigned ties = 0, pruned = 0;
+#pragma unroll
+                        for (int u = 0; u < kBoxAhead; ++u)
+                            ties |= (ok[u] && dsq[u] == r2) ? 1u << u : 0u;
+#pragma unroll 1
+                        for (int v = 0; v < kBoxAhead; ++v) {
+                            if (!((ties >> v) & 1))
+                                continue;
+                            int r = row0;
+#pragma unroll
+                            for (int u = 0; u < kBoxAhead; ++u)
+                                r = u == v ? row[u] : r;
+                            if (!(fabs(X[r] - q0) >= ti.range || fabs(Y[r] - q1) >= ti.range ||
+                                  (ND == 3 && fabs(Z[r] - q2) >= ti.range)))
+                                continue;
+                            if (!TREES)
+                                tie = true;
+                            else if (!walk_reaches<ND>(nodes + ti.node0, rownode[r], ti.range, q0, q1, q2))
+                                pruned |= 1u << v;
+                        }
+#pragma unroll
+                        for (int u = 0; u < kBoxAhead; ++u)
+                            ok[u] = ok[u] && !((pruned >> u) & 1);
+                    }
+#pragma unroll
+                    for (int u = 0; u < kBoxAhead; ++u)
+                        put(u);
                 }
             }
         }
@@ -689,7 +727,7 @@ __device__ inline int box_search(const TypeInfo& ti, const LocBox* __restrict__ 
     return n;
 }
 
-template <bool FILL>
+template <bool FILL, bool TREES>
 __global__ void __launch_bounds__(256) loc_box_kernel(int ni, int nj, const double* __restrict__ qxyz,
                                                       const unsigned char* __restrict__ isglobal,
                                                       const unsigned char* __restrict__ visible,
@@ -732,9 +770,9 @@ __global__ void __launch_bounds__(256) loc_box_kernel(int ni, int nj, const doub
             int* wid = FILL ? ids + o : nullptr;
             double* wlc = FILL ? lc + o : nullptr;
             n = ti.ndim == 3
-                    ? box_search<3, FILL>(ti, boxes, xyz, nrow, status, nodes, rownode, q, wid, wlc, wsd, wsi, tie)
-                    : box_search<2, FILL>(ti, boxes, xyz, nrow, status, nodes, rownode, q, wid, wlc, wsd, wsi, tie);
-            if (!FILL && __ballot(tie) && lane == 0)
+                    ? box_search<3, FILL, TREES>(ti, boxes, xyz, nrow, status, nodes, rownode, q, wid, wlc, wsd, wsi, tie)
+                    : box_search<2, FILL, TREES>(ti, boxes, xyz, nrow, status, nodes, rownode, q, wid, wlc, wsd, wsi, tie);
+            if (!FILL && !TREES && __ballot(tie) && lane == 0)
                 atomicExch(tieflag, 1);
         }
     }
@@ -941,14 +979,14 @@ hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, con
     constexpr long long per = (1LL << 24) / (8 * kBoxRun) - 1;
     for (long long r0 = 0; r0 < rounds; r0 += per) {
         const dim3 grid((unsigned)(round * std::min(per, rounds - r0)));
-        if (ids == nullptr)
-            hipLaunchKernelGGL(loc_box_kernel<false>, grid, dim3(256), 0, s, ni, nj, qxyz, isglobal, visible, types,
-                               ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc,
-                               tieflag, (unsigned)r0);
+        const auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, ni, nj, qxyz, isglobal, visible, types, ntypes, boxes, xyz,
+                               nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc, tieflag, (unsigned)r0);
+        };
+        if (nodes == nullptr)
+            ids == nullptr ? launch(loc_box_kernel<false, false>) : launch(loc_box_kernel<true, false>);
         else
-            hipLaunchKernelGGL(loc_box_kernel<true>, grid, dim3(256), 0, s, ni, nj, qxyz, isglobal, visible, types,
-                               ntypes, boxes, xyz, nrow, status, obsids, nodes, rownode, counts, offsets, ids, lc,
-                               tieflag, (unsigned)r0);
+            ids == nullptr ? launch(loc_box_kernel<false, true>) : launch(loc_box_kernel<true, true>);
     }
     return hipGetLastError();
 }
