@@ -456,6 +456,9 @@ int ensure_trees(enkfg_ctx* c)
     std::vector<int> rowof((size_t)std::max(c->nobs, 1), -1);
     for (int r = 0; r < c->nobs; ++r)
         rowof[(size_t)c->perm[(size_t)r]] = r;
+    std::vector<double> soa(3 * c->nsearch);   // coordinates of the rows, as enkfg_set_obs formed them
+    if (c->nsearch > 0)
+        HIPCHECK(c, hipMemcpy(soa.data(), c->d_xyz.p, soa.size() * sizeof(double), hipMemcpyDeviceToHost));
     std::vector<KdNode> dnodes(c->nsearch);
     std::vector<int> noderow(c->nsearch), rownode(c->nsearch);   // (a type's nodes are counted from its first)
     for (size_t t = 0; t < c->tinfo.size(); ++t) {
@@ -464,8 +467,10 @@ int ensure_trees(enkfg_ctx* c)
         std::sort(ids.begin(), ids.end());
         std::vector<double> xyz(3 * ids.size());
         for (size_t k = 0; k < ids.size(); ++k)
-            obs_coords(c, ids[k], c->types[t].geographic != 0, &xyz[3 * k]);
+            for (int d = 0; d < 3; ++d)
+                xyz[3 * k + d] = soa[d * c->nsearch + rowof[(size_t)ids[k]]];
         std::vector<BuildNode> nodes;
+        nodes.reserve(ids.size());
         build_tree(xyz, ti.ndim, ids, nodes);
         if ((int)nodes.size() != ti.nnode)
             return fail(c, ENKFG_ERR_ARG, "internal: kd-tree of obstype %d is incomplete", (int)t);
@@ -511,7 +516,7 @@ hipError_t fill_ordered(enkfg_ctx* c, bool nlobsmax)
 // The lists of `node` and of its neighbours in the reference's order, in a
 // buffer of their own: the calc's lists stay as they are.  A walk is a
 // thread's serial chain and takes about as long for a thousand nodes as for
-// one (12 ms for 9 nodes of 200 x 240 cells; 540x801 cells: 17 ms for 1,024
+// one (5.7 ms for 9 nodes of 200 x 240 cells; 540x801 cells: 9 ms for 1,024
 // nodes, 31 for all 48,060), so the first run takes kOrderRun nodes and each
 // further one eight times as many, for callers that read the whole grid.
 int order_run(enkfg_ctx* c, int node)
@@ -536,11 +541,12 @@ int order_run(enkfg_ctx* c, int node)
     const long long off0 = o[0] / 8 * 8;   // (whole bursts stay aligned)
     HIPCHECK(c, c->d_run_ids.reserve((size_t)(o[1] - off0) * sizeof(int)));
     HIPCHECK(c, c->d_run_lc.reserve((size_t)(o[1] - off0) * sizeof(double)));
-    HIPCHECK(c, launch_loc_fill_run(c->stream, node0, n, c->d_qxyz.as<double>(), c->d_glob.as<unsigned char>(),
-                                    c->lists_vis ? c->d_vis.as<unsigned char>() : nullptr, c->d_nodes.as<KdNode>(),
-                                    c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt, c->d_status.as<short>(),
-                                    c->d_obsids.as<int>(), c->d_offsets.as<long long>(), off0, c->d_run_ids.as<int>(),
-                                    c->d_run_lc.as<double>()));
+    HIPCHECK(c, launch_loc_fill(c->stream, c->list_ni, c->list_nj, c->d_qxyz.as<double>(),
+                                c->d_glob.as<unsigned char>(), c->lists_vis ? c->d_vis.as<unsigned char>() : nullptr,
+                                c->d_nodes.as<KdNode>(), c->d_noderow.as<int>(), c->d_types.as<TypeInfo>(), nt,
+                                c->d_status.as<short>(), c->d_obsids.as<int>(), c->d_offsets.as<long long>(),
+                                c->d_run_ids.as<int>(), c->d_run_lc.as<double>(), nullptr, nullptr, nullptr, nullptr,
+                                node0, n, off0));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     c->run_node0 = node0;
     c->run_n = n;

@@ -69,16 +69,13 @@ hipError_t launch_loc_box(hipStream_t s, int ni, int nj, const double* qxyz, con
                           const double* xyz, size_t nrow, const short* status, const int* obsids,
                           const KdNode* nodes, const int* rownode, int* counts, int* tieflag,
                           const long long* offsets, int* ids, double* lc);
+// the lists in the reference's order: of all nodes, or of nodes node0 .. node0
+// + n - 1 alone with entry off0 (a multiple of 8) of all lists at ids[0], lc[0]
 hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
                            const unsigned char* visible, const KdNode* nodes, const int* noderow,
-                           const TypeInfo* types, int ntypes, const short* status, const int* obsids, const long long* offsets, int* ids,
-                           double* lc, const long long* rawoff, const int* raw, const int* srow, const double* sd2);
-// the lists of nodes node0 .. node0 + n - 1 alone (no NLOBSMAX type), entry
-// off0 (a multiple of 8) of all lists at ids[0], lc[0]
-hipError_t launch_loc_fill_run(hipStream_t s, int node0, int n, const double* qxyz, const unsigned char* isglobal,
-                               const unsigned char* visible, const KdNode* nodes, const int* noderow,
-                               const TypeInfo* types, int ntypes, const short* status, const int* obsids,
-                               const long long* offsets, long long off0, int* ids, double* lc);
+                           const TypeInfo* types, int ntypes, const short* status, const int* obsids,
+                           const long long* offsets, int* ids, double* lc, const long long* rawoff, const int* raw,
+                           const int* srow, const double* sd2, int node0 = 0, int n = 0, long long off0 = 0);
 hipError_t launch_scan_counts(hipStream_t s, const int* counts, long long* offsets, long long n, void* tmp,
                               size_t* tmp_bytes);
 

@@ -404,9 +404,17 @@ __global__ void __launch_bounds__(256) loc_sort_big_kernel(int nnode, const Type
 // stores from 64 threads walking different lists leave their cache lines
 // part-written, and such lines are written back to memory several times over
 // (174 against 105 ms per localisation of the 51x1500x1800 tile; runs of 4
-// gave 118 ms, of 16 106 ms).  Nodes node0 .. nodeend - 1; ids and lc start at
-// list entry off0 (a multiple of kLocBurst).
+// gave 118 ms, of 16 106 ms).  nnode nodes from node0; ids and lc start at list
+// entry off0 (a multiple of kLocBurst).
+//
+// Few lists (lanes > 0): `lanes` of them in a row per wavefront instead of a
+// tile, so that they spread over kFillWaves wavefronts.  A wavefront's step
+// waits for the slowest of its lanes' loads, and a few wavefronts hide none of
+// it: 9 nodes of four types 13 -> 5.7 ms (512 to 8,192 wavefronts alike), 1,024
+// nodes 16.7 -> 8.9 ms (512: 10.7, 8,192: 7.4).
 constexpr int kLocBurst = 8;
+constexpr int kFillWaves = 2048;
+constexpr int kFillLanes = 8;   // beyond that, tiles
 
 __global__ void __launch_bounds__(64) loc_fill_kernel(int nnode, int ni, const double* __restrict__ qxyz,
                                                        const unsigned char* __restrict__ isglobal,
@@ -419,14 +427,20 @@ __global__ void __launch_bounds__(64) loc_fill_kernel(int nnode, int ni, const d
                                                        const long long* __restrict__ offsets, int* __restrict__ ids,
                                                        double* __restrict__ lc, const long long* __restrict__ rawoff,
                                                        const int* __restrict__ raw, const int* __restrict__ srow,
-                                                       const double* __restrict__ sd2, int node0, int nodeend, long long off0)
+                                                       const double* __restrict__ sd2, int node0, long long off0, int lanes)
 {
     int t, node;
-    if (!thread_node(nnode, ni, ntypes, t, node))
-        return;
+    if (lanes == 0) {
+        if (!thread_node(nnode, ni, ntypes, t, node))
+            return;
+    } else {
+        const long long it = (long long)blockIdx.x * lanes + threadIdx.x;
+        if ((int)threadIdx.x >= lanes || it >= (long long)nnode * ntypes)
+            return;
+        t = (int)(it / nnode);
+        node = (int)(it - (long long)t * nnode);
+    }
     node += node0;
-    if (node >= nodeend)
-        return;
     double q[3] = {qxyz[3 * (size_t)node], qxyz[3 * (size_t)node + 1], qxyz[3 * (size_t)node + 2]};
     const bool glob = isglobal[node] != 0;
     const TypeInfo& ti = types[t];
@@ -906,33 +920,25 @@ hipError_t launch_loc_nlobsmax(hipStream_t s, int ni, int nj, const double* qxyz
 
 hipError_t launch_loc_fill(hipStream_t s, int ni, int nj, const double* qxyz, const unsigned char* isglobal,
                            const unsigned char* visible, const KdNode* nodes, const int* noderow,
-                            const TypeInfo* types, int ntypes,
-                           const short* status, const int* obsids, const long long* offsets, int* ids, double* lc,
-                           const long long* rawoff, const int* raw, const int* srow, const double* sd2)
+                           const TypeInfo* types, int ntypes, const short* status, const int* obsids,
+                           const long long* offsets, int* ids, double* lc, const long long* rawoff, const int* raw,
+                           const int* srow, const double* sd2, int node0, int n, long long off0)
 {
-    const long long nt = (long long)ni * nj * ntypes;
+    const bool all = n == 0;
+    const long long nn = all ? (long long)ni * nj : n, nt = nn * ntypes;
     if (nt <= 0)
-        return hipSuccess;
-    hipLaunchKernelGGL(loc_fill_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
-                       visible, nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, rawoff, raw, srow, sd2,
-                       0, ni * nj, 0LL);
-    return hipGetLastError();
-}
-
-hipError_t launch_loc_fill_run(hipStream_t s, int node0, int n, const double* qxyz, const unsigned char* isglobal,
-                               const unsigned char* visible, const KdNode* nodes, const int* noderow,
-                               const TypeInfo* types, int ntypes, const short* status, const int* obsids,
-                               const long long* offsets, long long off0, int* ids, double* lc)
-{
-    if (n <= 0 || ntypes <= 0)
         return hipSuccess;
     if (off0 % kLocBurst != 0)
         return hipErrorInvalidValue;
-    // rows of eight nodes: a tile of thread_node is 64 nodes of the run
-    const int nj = (n + 7) / 8;
-    hipLaunchKernelGGL(loc_fill_kernel, walk_grid(8, nj, ntypes), dim3(64), 0, s, 8 * nj, 8, qxyz, isglobal, visible,
-                       nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, nullptr, nullptr, nullptr,
-                       nullptr, node0, node0 + n, off0);
+    const int lanes = (int)std::min<long long>((nt + kFillWaves - 1) / kFillWaves, 64);
+    if (all && lanes > kFillLanes)
+        hipLaunchKernelGGL(loc_fill_kernel, walk_grid(ni, nj, ntypes), dim3(64), 0, s, ni * nj, ni, qxyz, isglobal,
+                           visible, nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc, rawoff, raw, srow,
+                           sd2, 0, 0LL, 0);
+    else
+        hipLaunchKernelGGL(loc_fill_kernel, dim3((unsigned)((nt + lanes - 1) / lanes)), dim3(64), 0, s, (int)nn, ni,
+                           qxyz, isglobal, visible, nodes, noderow, types, ntypes, status, obsids, offsets, ids, lc,
+                           rawoff, raw, srow, sd2, node0, off0, lanes);
     return hipGetLastError();
 }
 
