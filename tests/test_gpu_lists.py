@@ -105,3 +105,21 @@ def test_a_refused_call_leaves_the_lists():
         assert call(E.h, None) != 0
     assert len(E.local_counts()) == P.node_lon.size
     E.close()
+
+
+@pytest.mark.parametrize("nj,ni", [(1, 3), (37, 61), (60, 70), (97, 101)])
+def test_lists_of_every_grid_size(nj, ni):
+    """The walk takes one list a wavefront, several, or tiles of nodes (beyond
+    16,384 lists): lists of enkfg_localise and of a run after a calc, two
+    obstypes, at the grid's corners and in between."""
+    print("case lists %d x %d nodes" % (nj, ni), flush=True)
+    P, E, ob = setup(profiles=40)
+    assert len(P.obstypes) == 2
+    lon, lat = np.meshgrid(np.linspace(P.lon.min() - 0.5, P.lon.max(), ni), np.linspace(P.lat.min(), P.lat.max() + 0.5, nj))
+    nn = nj * ni
+    nodes = sorted({0, ni - 1, nn // 2, nn - ni, nn - 1, *range(0, nn, 97)} | set(range(max(0, nn - 9), nn)))
+    E.localise(lon, lat)
+    check_lists(E, ob, lon, lat, nodes)
+    E.calc_transforms(lon, lat)
+    check_lists(E, ob, lon, lat, nodes)
+    E.close()
