@@ -13,7 +13,7 @@
 // m ..) is kept the identity in Y and Z, as it is in M: scaled with the rest, it
 // would enter the determinants, whose root is of order 2m, and for m <= 7 mu
 // runs away.  Each inverse is combined tile by tile as it is formed.  The first step
-// needs one inverse (Z_0 = I; it gives w, dfs and srf too), the last one
+// needs one inverse (Z_0 = I; it gives w, dfs = tr(M^-1 G) and srf too), the last one
 // Y_k^-1 only.  Once a step changes Z by less than 1e-8 of its norm, one more
 // unscaled step is taken and is the last (the iteration converges
 // quadratically); no convergence in 60 steps is reported.
@@ -25,11 +25,10 @@
 // the workspace's traffic (130 KB an inverse).  For m = 96 about 14 inverses
 // a node.  Measured against the kernel before it (pivots swept one per
 // workgroup barrier, one five-wave workgroup per CU): 51x1500x1800 tile FP64
-// calc 1,909 -> 561 ms; 4,050 nodes, m = 96: 21.0 -> 4.3 ms; 2,278 nodes, m =
-// 24: 0.61 -> 0.22 ms.  m > 96 had iterates in memory and Gauss-Jordan
-// inverses of up to 2 KB of spills a lane; it takes the same path now (488
-// and 980 B of spills at MT = 9 and 10, 164 at 6: tile_waves).  Counters on the
-// tile: matrix cores busy 41%, VALU issue 26%.
+// calc 1,909 -> 550 ms; 4,050 nodes, m = 96: 21.0 -> 3.9 ms; 2,278 nodes, m =
+// 24: 0.61 -> 0.23 ms.  m > 96 had iterates in memory and Gauss-Jordan
+// inverses of up to 2 KB of spills a lane; it takes the same path now (136 B
+// of spills a lane at MT = 6, 440 and 964 at 9 and 10: tile_waves).
 #include <algorithm>
 
 #include "enkfg_internal.h"
@@ -93,10 +92,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
         __syncthreads();
 
         // Y_0 = M
-        double trg;
+        double trg, g2;
         {
             tile4 x[tri_count(MT)];
-            trg = load_tiles<MT, false>(a, bnode, node, 0, a.nseg, lane, x);
+            trg = load_tiles<MT, false, true>(a, bnode, node, 0, a.nseg, lane, x, &g2);
 #pragma unroll
             for (int f = 0; f < tri_count(MT); ++f)
 #pragma unroll
@@ -243,7 +242,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_wa
             if (first) {
                 trx = wave_sum(trx) - (double)(MP - m);
                 if (lane == 0) {
-                    const float fd = (float)((double)m - trx);   // m - tr(M^-1)
+                    // m - tr(M^-1) to m eps; where that shows, by the first two
+                    // terms of tr(G) - tr(G^2) + tr(G^3) - ..., to 1e-10
+                    const double dfs = (double)m - trx;
+                    const float fd = (float)(dfs > 1e-5 ? dfs : trg - g2);
                     a.pnlobs[(size_t)nt * a.nnode + node] = p;
                     a.pdfs[(size_t)nt * a.nnode + node] = fd;
                     a.psrf[(size_t)nt * a.nnode + node] = (float)(sqrt(trg / (double)fd) - 1.0);

@@ -288,7 +288,7 @@ __device__ __attribute__((always_inline)) inline void tile_inverse(const tile4* 
 // SIMD's 512 registers is 8 for each tile and what the kernel needs beside
 // them, which is more than the rest of the share for some MT: the DEnKF and
 // trace kernels spill 10 and 8 registers at MT = 6, 14 and 8 at 8, 206 and 130
-// at 9, 789 and 542 at 10, the ETKF kernel 24, 97, 97, 22, 32, 291 and 956 at
+// at 9, 789 and 542 at 10, the ETKF kernel 22, 99, 44, 24, 34, 304 and 780 at
 // 2, 3, 6, 7, 8, 9 and 10 (compiler's report).  Other counts for these have
 // not been measured.
 __host__ __device__ constexpr int tile_waves(int MT) { return MT <= 3 ? 4 : (MT <= 6 ? 2 : 1); }
@@ -326,10 +326,10 @@ __device__ __attribute__((always_inline)) inline void read_tiles(const double* g
 }
 
 // x <- I + the Gram matrices of segments s0 .. s1 - 1 (ONE: s0) of batch node bnode;
-// returns the trace of the Gram matrix
-template <int MT, bool ONE>
+// returns the trace of the Gram matrix G (NORM2: norm2 <- |G|^2)
+template <int MT, bool ONE, bool NORM2 = false>
 __device__ __attribute__((always_inline)) inline double load_tiles(const CalcArgs& a, int bnode, int node, int s0,
-                                                                   int s1, int lane, tile4* x)
+                                                                   int s1, int lane, tile4* x, double* norm2 = nullptr)
 {
     constexpr int NT = tri_count(MT);
     // the first segment's tiles are loaded straight into x, all at once; the
@@ -366,6 +366,17 @@ __device__ __attribute__((always_inline)) inline double load_tiles(const CalcArg
 #pragma unroll
         for (int f = 0; f < NT; ++f)
             tile_pin(x[f]);
+    }
+    if constexpr (NORM2) {
+        double d = 0.0, o = 0.0;   // of the diagonal tiles, and of the others
+        static_for<0, NT>([&](auto fc) {
+            constexpr int f = fc;
+            double& v = tri_I(MT, f) == tri_J(MT, f) ? d : o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                v = fma(x[f][r], x[f][r], v);
+        });
+        *norm2 = wave_sum(d + 2.0 * o);
     }
     double tr = 0.0;
 #pragma unroll

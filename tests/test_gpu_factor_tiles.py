@@ -85,3 +85,33 @@ def test_factor_etkf_sizes(m, errscale):
         assert np.abs(T64[k] - (V / np.sqrt(lam)) @ V.T).max() <= tol
         wr = (V / lam) @ (V.T @ b)
         assert np.abs(w64[k] - wr).max() <= tol * np.abs(wr).max() + 4 * m * eps * (np.abs(A) @ np.abs(s[ids] * lc)).max()
+
+
+@pytest.mark.parametrize("m", [24, 96, 100, 144])
+@pytest.mark.parametrize("errscale", [1e3, 1e5, 3e7])
+def test_factor_etkf_weak_observations(m, errscale):
+    """dfs = tr(M^-1 G) and srf = sqrt(tr(G) / dfs) - 1 of ETKF columns whose
+    observations hardly constrain them: dfs down to 1e-14, far below the
+    rounding of m - tr(M^-1).  Both are FP32 results; G has the rounding of
+    FP64 sums.  srf is tiny there: it is compared as sqrt(tr(G) / dfs)."""
+    print("case etkf weak m=%d errscale=%g" % (m, errscale), flush=True)
+    P = synth.make_problem(seed=m, nmem=m, nobs=700, nj=16, ni=20, nk=3, locrad=60.0, stride=4, profiles=40)
+    estd = (P.obs_estd * errscale).astype(np.float32)
+    ob = O.OracleObs(P.obstypes, P.obs_type, P.obs_lon, P.obs_lat, estd)
+    S, s = O.standardise(m, ob, P.HA, P.innov)
+    E = enkfg.Engine(m, scheme=enkfg.SCHEME_ETKF)
+    E.set_obstypes(P.obstypes)
+    E.set_obs(P.obs_type, P.obs_status, P.obs_lon, P.obs_lat, estd)
+    E.set_S(P.HA, P.innov, standardised=False)
+    E.calc_transforms(P.node_lon, P.node_lat, stride=P.stride)
+    _, pd, ps = E.diag()
+    E.close()
+    pd, ps = pd.reshape(len(P.obstypes) + 1, -1)[-1], ps.reshape(len(P.obstypes) + 1, -1)[-1]
+    for k, (lo, la) in enumerate(zip(P.node_lon.ravel(), P.node_lat.ravel())):
+        ids, lc = ob.findlocal(lo, la)
+        A = S[:, ids].astype(np.float64) * lc
+        # the eigenvalues of G: the squares of A's singular values
+        lam = np.linalg.svd(A, compute_uv=False) ** 2
+        dfs = (lam / (1.0 + lam)).sum()
+        assert abs(pd[k] - dfs) <= 4 * np.finfo(np.float32).eps * dfs
+        assert abs(ps[k] + 1.0 - np.sqrt(lam.sum() / dfs)) <= 8 * np.finfo(np.float32).eps * np.sqrt(lam.sum() / dfs)
