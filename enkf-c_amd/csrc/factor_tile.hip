@@ -29,7 +29,7 @@
 // ms; 96 + 48 members on 8,000 nodes 10.2 -> 5.4 ms; m = 130, EnOI 2.9 -> 1.4
 // ms.  For MT >= 7 one wavefront per SIMD holds its tiles in 512 registers;
 // some MT spill (tile_waves).  Counters on the tile, the kernels alone: matrix
-// cores busy 51% of a trace launch and 29% of a node launch, VALU issue 39%
+// cores busy 51% of a trace launch and 30% of a node launch, VALU issue 38%
 // and 27%.
 #include "enkfg_internal.h"
 #include "gram_layout.h"

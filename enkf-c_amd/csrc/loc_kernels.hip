@@ -36,7 +36,7 @@
 // loads beyond L2 and by the depth of the trees (walking and compacting the
 // lists took 100 ms with the observations in random order, 991 ms in
 // enkf_prep order); the box search, counting and filling, by FP64 issue (a
-// leaf's distances twice, the tapers once) at 17.3 ms in either order.  On
+// leaf's distances twice, the tapers once) at 17.5 ms in either order.  On
 // 200 x 240 cells and 9 nodes it takes 0.14 ms against 13 ms: a walk's
 // dependent loads are one chain per thread, a box search's steps load 64
 // boxes or 256 observations each.
