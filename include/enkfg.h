@@ -156,9 +156,11 @@ int enkfg_sync(enkfg_ctx* ctx);
 int enkfg_set_obstypes(enkfg_ctx* ctx, int ntypes, const enkfg_obstype* types);
 
 /* obs_read() output plus obs_createkdtrees() (observations.c:1616): per
- * non-stats-only obstype, obs with status OK are inserted, in ascending index
- * order, into a kd-tree over 3D chord coordinates (geographic types) or
- * (lon, lat).  lon/lat are the float obs coordinates of observations.h:67-68. */
+ * non-stats-only obstype, the obs with status OK are those that are searched,
+ * by 3D chord coordinates (geographic types) or (lon, lat).  lon/lat are the
+ * float obs coordinates of observations.h:67-68.  They are sorted for the
+ * calc's search here; the reference's kd-trees, into which it inserts them in
+ * ascending index order, are built by the first call that needs them. */
 int enkfg_set_obs(enkfg_ctx* ctx, int nobs, const short* type, const short* status, const float* lon, const float* lat, const float* estd);
 
 /* H operators of the obs types (calc/allhs.c:30-44) that enkfg_calc_HE
